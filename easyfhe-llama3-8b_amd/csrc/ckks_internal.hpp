@@ -183,6 +183,21 @@ __device__ __forceinline__ u64 mul_mod(u64 a, u64 b, const ModQ &M) {
   return barrett(__umul64hi(a, b), a * b, M);
 }
 
+// x = hi 2^64 + lo < q 2^64: x 2^-64 mod q in [0, 2q)
+__device__ __forceinline__ u64 redc_lazy(u64 hi, u64 lo, u64 q, u64 qinv) {
+  const u64 m = lo * qinv;
+  return hi + __umul64hi(m, q) + (lo != 0 ? 1 : 0);
+}
+
+// a b mod q in [0, 3q) for a, b < q (Barrett without its last subtractions)
+__device__ __forceinline__ u64 mul_lazy(u64 a, u64 b, const ModQ &M) {
+  const u64 hi = __umul64hi(a, b), lo = a * b;
+  const u32 k = M.k;
+  const u64 xs = (hi << (65 - k)) | (lo >> (k - 1));
+  const u64 ph = __umul64hi(xs, M.mu), pl = xs * M.mu;
+  return lo - ((ph << (63 - k)) | (pl >> (k + 1))) * M.q;
+}
+
 __device__ __forceinline__ u64 to_mont(u64 a, const ModQ &M) {
   return redc(__umul64hi(a, M.r2), a * M.r2, M.q, M.qinv);
 }

@@ -237,25 +237,130 @@ __global__ __launch_bounds__(TPB) void k_ntt_inv_high(Batch dst, int logN, int l
 // the +1 per 16 keeps 16-apart columns in distinct banks.
 // ===========================================================================
 
-__device__ __forceinline__ u64 shoup_lazy(u64 a, u64 w, u64 ws, u64 q) {
-  return a * w - __umul64hi(a, ws) * q;  // in [0, 2q) for any a < 2^64
+// Lazy 64-bit arithmetic of the N = 2^16 transforms (primes 2^45 <= q < 2^60).
+// Issue bounds the butterflies: every 32-bit multiply, multiply-add and add
+// is one full-rate instruction on gfx950, a 64-bit conditional subtraction
+// about 6 lane-cycles.  So words run up to 16q < 2^64 and are reduced by a
+// multiply once in three stages, the quotient is short by up to 2 (two
+// multiplies and their carries less), and the sum x + wY is formed inside the
+// product's multiply-adds: 15.5 lane-cycles a butterfly in a register loop,
+// against 26.9 with an exact quotient and a conditional subtraction in every
+// stage (a split of Y at 31 bits with 7 multiplies in place of 9: 18.6).
+// Forward low pass of 16 ciphertexts at 13 + 8 limbs of 59 and 60 bits: 278 ->
+// 233 us; fused key product 334 -> 294 us.
+// Constants of one prime:
+struct LazyQ {
+  u64 q, nq;  // q, -q mod 2^64
+  u32 mu;     // floor(2^64 / q)
+  u32 mus;    // floor(2^(64 + sh) / q) < 2^32
+  u32 sh;     // bit length of q - 33
+};
+__device__ __forceinline__ LazyQ lazy_q(u64 q, u64 barrett_mu, u32 k) {
+  // barrett_mu = floor(2^(2 k) / q)
+  return LazyQ{q, 0 - q, (u32)(barrett_mu >> (2 * k - 64)), (u32)(barrett_mu >> (k - 31)),
+               k - 33};
+}
+__device__ __forceinline__ LazyQ lazy_q(const ModQ &M) { return lazy_q(M.q, M.mu, M.k); }
+
+// floor(a b / 2^64) less 0, 1 or 2: the low halves' product and the two
+// carries into the upper word are left out
+__device__ __forceinline__ u64 umul64hi_low(u64 a, u64 b) {
+  const u32 a0 = (u32)a, a1 = (u32)(a >> 32), b0 = (u32)b, b1 = (u32)(b >> 32);
+  return (u64)a1 * b1 + __umulhi(a0, b1) + __umulhi(a1, b0);
 }
 
-// Cooley-Tukey: X, Y in [0, 4q) -> X + wY, X - wY in [0, 4q)
-__device__ __forceinline__ void ct_bfly(u64 &X, u64 &Y, u64 w, u64 ws, u64 q, u64 q2) {
-  const u64 x = csub(X, q2);
-  const u64 t = shoup_lazy(Y, w, ws, q);
-  X = x + t;
-  Y = x - t + q2;
+// x + t mod 2^64 with t = a w mod q in [0, 4q), any a < 2^64, ws = floor(w
+// 2^64 / q): Shoup's quotient is at most 1 below a w / q, umul64hi_low at
+// most 2 below the quotient.  x and the product's correction enter the
+// multiply-adds of the low halves, so neither costs an addition of its own.
+__device__ __forceinline__ u64 shoup_add(u64 x, u64 a, u64 w, u64 ws, const LazyQ &Q) {
+  const u64 h = umul64hi_low(a, ws);
+  return x + a * w + h * Q.nq;
 }
 
-// Gentleman-Sande: X, Y in [0, 2q) -> X + Y, (X - Y) w in [0, 2q)
-__device__ __forceinline__ void gs_bfly(u64 &X, u64 &Y, u64 w, u64 ws, u64 q, u64 q2) {
-  u64 sum = X + Y;
-  sum = csub(sum, q2);
-  const u64 d = X - Y + q2;
-  X = sum;
-  Y = shoup_lazy(d, w, ws, q);
+// x < 2^64 to [0, (2 + 2^-13) q): the quotient from the upper word is at most
+// 1 + 2^-13 below x / q before its own rounding
+__device__ __forceinline__ u64 lazy_reduce(u64 x, const LazyQ &Q) {
+  const u32 h = __umulhi((u32)(x >> 32), Q.mu);
+  return x + (u64)h * Q.nq;
+}
+
+// x < 2^64 to [0, q): with sh more bits of 2^64 / q the quotient is less than
+// 2 below x / q, one conditional subtraction is left
+__device__ __forceinline__ u64 lazy_canon(u64 x, const LazyQ &Q) {
+  const u32 h = __umulhi((u32)(x >> 32), Q.mus) >> Q.sh;
+  return csub(x + (u64)h * Q.nq, Q.q);
+}
+
+// Cooley-Tukey butterfly: (X, Y) -> (X + wY, X - wY + 4q), both below X + 4q.
+// Y may be any word; X < 12q (2^64 > 16q) with RED false, any word with RED
+// true (X is reduced first: both results below (6 + 2^-13) q).
+template <bool RED>
+__device__ __forceinline__ void ct_bfly(u64 &X, u64 &Y, u64 w, u64 ws, const LazyQ &Q) {
+  const u64 x = RED ? lazy_reduce(X, Q) : X;
+  const u64 s = shoup_add(x, Y, w, ws, Q);
+  Y = ((x << 1) + 4 * Q.q) - s;
+  X = s;
+}
+
+// Gentleman-Sande butterfly: X, Y <= 8q -> X + Y, (X - Y) w in [0, 4q)
+__device__ __forceinline__ void gs_bfly(u64 &X, u64 &Y, u64 w, u64 ws, const LazyQ &Q) {
+  const u64 d = (X + 8 * Q.q) - Y;
+  X = X + Y;
+  Y = shoup_add(0, d, w, ws, Q);
+}
+
+// Where the four stages of an inverse round reduce (red[st][k]: word k before
+// stage st, red[4]: after the last): every word enters with bound `in` (in
+// units of q), stage st pairs k with k + 2^st, a sum adds its operands'
+// bounds, a product is below 4q, and a word above 8q is reduced (to below 3q)
+// before its butterfly and, unless the round is the last, after the round.
+struct InvPlan {
+  bool red[5][16];
+};
+constexpr InvPlan inv_plan(int in, bool last) {
+  InvPlan p{};
+  int b[16] = {};
+  for (int k = 0; k < 16; k++) b[k] = in;
+  for (int st = 0; st < 4; st++) {
+    const int half = 1 << st;
+    for (int k = 0; k < 16; k++) {
+      p.red[st][k] = b[k] > 8;
+      if (b[k] > 8) b[k] = 3;
+    }
+    for (int k = 0; k < 16; k++) {
+      if (k & half) continue;
+      b[k] = b[k] + b[k + half];
+      b[k + half] = 4;
+    }
+  }
+  for (int k = 0; k < 16; k++) p.red[4][k] = !last && b[k] > 8;
+  return p;
+}
+
+// The four stages of an inverse round on words in [0, IN q): stage st pairs
+// bit st of k, tw(st, k) gives the twiddle index of the pair (k, k + 2^st).
+// Output in [0, 8q], or any word with LAST.
+template <int IN, bool LAST, typename F>
+__device__ __forceinline__ void u64_inv_round(u64 (&x)[16], const u64 *__restrict__ W,
+                                              const u64 *__restrict__ Ws, const LazyQ &Q, F tw) {
+  constexpr InvPlan plan = inv_plan(IN, LAST);
+#pragma unroll
+  for (int st = 0; st < 4; st++) {
+    const int half = 1 << st;
+#pragma unroll
+    for (int k = 0; k < 16; k++)
+      if (plan.red[st][k]) x[k] = lazy_reduce(x[k], Q);
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+      if (k & half) continue;
+      const int ti = tw(st, k);
+      gs_bfly(x[k], x[k + half], W[ti], Ws[ti], Q);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 16; k++)
+    if (plan.red[4][k]) x[k] = lazy_reduce(x[k], Q);
 }
 
 __device__ __forceinline__ int lds16(int r, int c) { return r * 272 + c + (c >> 4); }
@@ -355,12 +460,13 @@ __device__ __forceinline__ void md_sub_load(const MDCombine &md, int item2, int 
   }
 }
 
-// (dbl ? 2 r : r) - s + sc with r = (a - y) P^-1 + d amul (apply_post's terms)
+// (dbl ? 2 r : r) - s + sc with r = (a - y) P^-1 + d amul (apply_post's terms);
+// y < 8q
 __device__ __forceinline__ void md_store(const MDCombine &md, int item2, int limb, u32 e, u64 y,
                                          const MDPrefetch &pf, u64 a, u64 d, u64 s, u64 q) {
   const int item = item2 >> 1, comp = item2 & 1;
   const size_t N = 65536;
-  u64 r = shoup_mul(sub_mod(a, y, q), pf.pinv, pf.pinvs, q);
+  u64 r = shoup_mul(a + 8 * q - y, pf.pinv, pf.pinvs, q);
   if (md.amul) d = shoup_mul(d, pf.am, pf.ams, q);
   r = add_mod(r, d, q);
   if (md.post.dbl) r = add_mod(r, r, q);
@@ -370,115 +476,93 @@ __device__ __forceinline__ void md_store(const MDCombine &md, int item2, int lim
   o[(size_t)limb * N + e] = r;
 }
 
-// High pass, 64-bit body: x[k] = word c + 4096 k of one column, stages on
-// bits 15..12 (k bits 3..0); the twiddle of stage st and pair k is
+// The stages of a 64-bit forward transform; bounds in units of q, R: the
+// stage reduces its X operands first (2^64 > 16q, a stage adds at most 4q).
+//   high pass (bits 15..12): in < 4q:  8, 12, 16, R 6+
+//   low pass:                in < 8q:
+//     round Z (11..8):  12, 16, R 6+, 10+
+//     round A (7..4):   14+, R 6+, 10+, 14+
+//     round B (3..0):   R 6+, 10+, 14+, R 6+ (below 7q)
+// High pass: x[k] = word c + 4096 k of one column, stages on bits 15..12 (k
+// bits 3..0); the twiddle of stage st and pair k is
 // psi_br[2^st + (k >> (4 - st))], the same for every column.
-__device__ __forceinline__ void u64_high_fwd(u64 (&x)[16], const u64 *__restrict__ W,
-                                             const u64 *__restrict__ Ws, u64 q, u64 q2) {
+template <int R0, int R1, typename F>
+__device__ __forceinline__ void u64_fwd_round(u64 (&x)[16], const u64 *__restrict__ W,
+                                              const u64 *__restrict__ Ws, const LazyQ &Q, F tw) {
 #pragma unroll
   for (int st = 0; st < 4; st++) {
     const int half = 8 >> st;
 #pragma unroll
     for (int k = 0; k < 16; k++) {
       if (k & half) continue;
-      const int ti = (1 << st) + (k >> (4 - st));
-      ct_bfly(x[k], x[k + half], W[ti], Ws[ti], q, q2);
+      const int ti = tw(st, k);
+      if (st == R0 || st == R1) ct_bfly<true>(x[k], x[k + half], W[ti], Ws[ti], Q);
+      else ct_bfly<false>(x[k], x[k + half], W[ti], Ws[ti], Q);
     }
   }
 }
 
-// inverse high pass on one column (lazy input, lazy output in [0, 2q))
+__device__ __forceinline__ void u64_high_fwd(u64 (&x)[16], const u64 *__restrict__ W,
+                                             const u64 *__restrict__ Ws, const LazyQ &Q) {
+  u64_fwd_round<3, 3>(x, W, Ws, Q, [](int st, int k) { return (1 << st) + (k >> (4 - st)); });
+}
+
+// inverse high pass on one column (input in [0, 8q], lazy output)
 __device__ __forceinline__ void u64_high_inv_stages(u64 (&x)[16], const u64 *__restrict__ W,
-                                                    const u64 *__restrict__ Ws, u64 q, u64 q2) {
-#pragma unroll
-  for (int st = 3; st >= 0; st--) {
-    const int half = 8 >> st;
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-      if (k & half) continue;
-      const int ti = (1 << st) + (k >> (4 - st));
-      gs_bfly(x[k], x[k + half], W[ti], Ws[ti], q, q2);
-    }
-  }
+                                                    const u64 *__restrict__ Ws, const LazyQ &Q) {
+  u64_inv_round<8, true>(x, W, Ws, Q, [](int st, int k) { return (8 >> st) + (k >> (st + 1)); });
 }
 
 // the inverse high pass, then x N^-1 to [0, q)
 __device__ __forceinline__ void u64_high_inv(u64 (&x)[16], const u64 *__restrict__ W,
                                              const u64 *__restrict__ Ws, u64 ni, u64 nis,
-                                             u64 q, u64 q2) {
-  u64_high_inv_stages(x, W, Ws, q, q2);
+                                             const LazyQ &Q) {
+  u64_high_inv_stages(x, W, Ws, Q);
 #pragma unroll
-  for (int k = 0; k < 16; k++) {
-    const u64 v = shoup_lazy(x[k], ni, nis, q);
-    x[k] = csub(v, q);
-  }
+  for (int k = 0; k < 16; k++) x[k] = shoup_mul(x[k], ni, nis, Q.q);
 }
 
 // Round Z of the forward low pass: x[k] = word t + 256 k of tile `tile`
 // (position j = 4096 tile + 256 k + t), stages on bits 11..8 (k bits 3..0);
 // twiddle index (N >> (b + 1)) + (j >> (b + 1)) does not depend on t.
 __device__ __forceinline__ void u64_low_round_z(u64 (&x)[16], const u64 *__restrict__ W,
-                                                const u64 *__restrict__ Ws, int tile, u64 q,
-                                                u64 q2) {
-#pragma unroll
-  for (int st = 0; st < 4; st++) {
-    const int b = 11 - st, half = 8 >> st;
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-      if (k & half) continue;
-      const int ti = (65536 >> (b + 1)) + ((tile * 4096 + 256 * k) >> (b + 1));
-      ct_bfly(x[k], x[k + half], W[ti], Ws[ti], q, q2);
-    }
-  }
+                                                const u64 *__restrict__ Ws, int tile,
+                                                const LazyQ &Q) {
+  u64_fwd_round<2, 2>(x, W, Ws, Q, [&](int st, int k) {
+    const int b = 11 - st;
+    return (65536 >> (b + 1)) + ((tile * 4096 + 256 * k) >> (b + 1));
+  });
 }
 
 // inverse round Z: stages on bits 8..11, same positions as round Z
 __device__ __forceinline__ void u64_inv_round_z(u64 (&x)[16], const u64 *__restrict__ W,
-                                                const u64 *__restrict__ Ws, int tile, u64 q,
-                                                u64 q2) {
-#pragma unroll
-  for (int b = 8; b < 12; b++) {
-    const int half = 1 << (b - 8);
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-      if (k & half) continue;
-      const int ti = (65536 >> (b + 1)) + ((tile * 4096 + 256 * k) >> (b + 1));
-      gs_bfly(x[k], x[k + half], W[ti], Ws[ti], q, q2);
-    }
-  }
+                                                const u64 *__restrict__ Ws, int tile,
+                                                const LazyQ &Q) {
+  u64_inv_round<8, false>(x, W, Ws, Q, [&](int st, int k) {
+    const int b = 8 + st;
+    return (65536 >> (b + 1)) + ((tile * 4096 + 256 * k) >> (b + 1));
+  });
 }
 
 // Rounds of the forward low pass on one thread's 16 words of global row
 // `row` (of 256): A on columns c0 + 16 k (bits 7..4), B on columns 16 c0 + j
-// (bits 3..0); values in [0, 4q)
+// (bits 3..0); values below 7q after B
 __device__ __forceinline__ void u64_low_round_a(u64 (&x)[16], const u64 *__restrict__ W,
-                                                const u64 *__restrict__ Ws, int row, u64 q,
-                                                u64 q2) {
-#pragma unroll
-  for (int st = 0; st < 4; st++) {
-    const int b = 7 - st, half = 8 >> st;
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-      if (k & half) continue;
-      const int ti = (65536 >> (b + 1)) + ((row * 256 + 16 * k) >> (b + 1));
-      ct_bfly(x[k], x[k + half], W[ti], Ws[ti], q, q2);
-    }
-  }
+                                                const u64 *__restrict__ Ws, int row,
+                                                const LazyQ &Q) {
+  u64_fwd_round<1, 1>(x, W, Ws, Q, [&](int st, int k) {
+    const int b = 7 - st;
+    return (65536 >> (b + 1)) + ((row * 256 + 16 * k) >> (b + 1));
+  });
 }
 
 __device__ __forceinline__ void u64_low_round_b(u64 (&x)[16], const u64 *__restrict__ W,
-                                                const u64 *__restrict__ Ws, int row, int c0, u64 q,
-                                                u64 q2) {
-#pragma unroll
-  for (int st = 4; st < 8; st++) {
-    const int b = 7 - st, half = 1 << b;
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-      if (j & half) continue;
-      const int ti = (65536 >> (b + 1)) + ((row * 256 + 16 * c0 + j) >> (b + 1));
-      ct_bfly(x[j], x[j + half], W[ti], Ws[ti], q, q2);
-    }
-  }
+                                                const u64 *__restrict__ Ws, int row, int c0,
+                                                const LazyQ &Q) {
+  u64_fwd_round<0, 3>(x, W, Ws, Q, [&](int st, int j) {
+    const int b = 3 - st;
+    return (65536 >> (b + 1)) + ((row * 256 + 16 * c0 + j) >> (b + 1));
+  });
 }
 
 // Round Z of tile `tile` from src (words t + 256 k), its result into the LDS
@@ -487,13 +571,13 @@ __device__ __forceinline__ void u64_low_round_b(u64 (&x)[16], const u64 *__restr
 __device__ __forceinline__ void u64_round_z_to_lds(u64 *__restrict__ sm,
                                                    const u64 *__restrict__ src,
                                                    const u64 *__restrict__ W,
-                                                   const u64 *__restrict__ Ws, int tile, u64 q,
-                                                   u64 q2) {
+                                                   const u64 *__restrict__ Ws, int tile,
+                                                   const LazyQ &Q) {
   const int t = threadIdx.x;
   u64 x[16];
 #pragma unroll
   for (int k = 0; k < 16; k++) x[k] = src[t + 256 * k];
-  u64_low_round_z(x, W, Ws, tile, q, q2);
+  u64_low_round_z(x, W, Ws, tile, Q);
 #pragma unroll
   for (int k = 0; k < 16; k++) sm[lds16(k, t)] = x[k];
 }
@@ -509,7 +593,7 @@ __device__ __forceinline__ void k_ntt16_fwd_low_body(u64 *__restrict__ lds, Batc
   u64 *sm = lds;
   const int limb = l_begin + blockIdx.z;
   const int p = prime_of(limb, q_limbs, L);
-  const u64 q = mods[p].q, q2 = 2 * q;
+  const LazyQ Q = lazy_q(mods[p]);
   const u64 *W = psi + ((size_t)p << 16);
   const u64 *Ws = psi_sh + ((size_t)p << 16);
   u64 *base = batch_ptr(dst, blockIdx.y) + ((size_t)limb << 16) + (size_t)blockIdx.x * 4096;
@@ -517,27 +601,26 @@ __device__ __forceinline__ void k_ntt16_fwd_low_body(u64 *__restrict__ lds, Batc
   const int row = blockIdx.x * 16 + rl;  // global row of 256
   MDPrefetch pf;
   if constexpr (COMBINE) md_load(md, blockIdx.y, limb, blockIdx.x * 4096 + rl * 256 + c0, pf);
-  u64_round_z_to_lds(sm, base, W, Ws, blockIdx.x, q, q2);
+  u64_round_z_to_lds(sm, base, W, Ws, blockIdx.x, Q);
   __syncthreads();
   u64 x[16];
   // round A: column = c0 + 16 k, stages on column bits 7..4; the thread
   // writes back the slots it read, which no other thread reads
 #pragma unroll
   for (int k = 0; k < 16; k++) x[k] = sm[lds16(rl, c0 + 16 * k)];
-  u64_low_round_a(x, W, Ws, row, q, q2);
+  u64_low_round_a(x, W, Ws, row, Q);
 #pragma unroll
   for (int k = 0; k < 16; k++) sm[lds16(rl, c0 + 16 * k)] = x[k];
   row_sync();
   // round B: column = 16 c0 + j, stages on column bits 3..0
 #pragma unroll
   for (int j = 0; j < 16; j++) x[j] = sm[lds16(rl, 16 * c0 + j)];
-  u64_low_round_b(x, W, Ws, row, c0, q, q2);
+  u64_low_round_b(x, W, Ws, row, c0, Q);
   // store through LDS so that adjacent lanes write adjacent words
   row_sync();
 #pragma unroll
-  for (int j = 0; j < 16; j++) {
-    sm[lds16(rl, 16 * c0 + j)] = csub(csub(x[j], q2), q);
-  }
+  for (int j = 0; j < 16; j++)
+    sm[lds16(rl, 16 * c0 + j)] = COMBINE ? x[j] : lazy_canon(x[j], Q);
   row_sync();
   if constexpr (COMBINE) {
     const u32 e0 = blockIdx.x * 4096 + rl * 256 + c0;
@@ -546,14 +629,14 @@ __device__ __forceinline__ void k_ntt16_fwd_low_body(u64 *__restrict__ lds, Batc
 #pragma unroll
     for (int k = 0; k < 16; k++)
       md_store(md, blockIdx.y, limb, e0 + 16 * k, sm[lds16(rl, c0 + 16 * k)], pf, pf.a[k],
-               pf.d[k], sv[k], q);
+               pf.d[k], sv[k], Q.q);
   } else {
 #pragma unroll
     for (int k = 0; k < 16; k++) base[rl * 256 + c0 + 16 * k] = sm[lds16(rl, c0 + 16 * k)];
   }
 }
 
-// inverse, bit positions 0..11 (first pass): input in [0, 2q), output lazy
+// inverse, bit positions 0..11 (first pass): input in [0, 2q), output in [0, 8q]
 __device__ __forceinline__ void k_ntt16_inv_low_body(u64 *__restrict__ lds, Batch src, Batch dst, int l_begin,
                                                        int q_limbs, int L,
                                                        const ModQ *__restrict__ mods,
@@ -563,7 +646,8 @@ __device__ __forceinline__ void k_ntt16_inv_low_body(u64 *__restrict__ lds, Batc
   u64 *sm = lds;
   const int limb = l_begin + blockIdx.z;
   const int p = prime_of(limb, q_limbs, L);
-  const u64 q = mods[p].q, q2 = 2 * q;
+  const ModQ M = mods[p];
+  const LazyQ Q = lazy_q(M);
   const u64 *W = ipsi + ((size_t)p << 16);
   const u64 *Ws = ipsi_sh + ((size_t)p << 16);
   const u64 *in = batch_ptr(src, blockIdx.y) + ((size_t)limb << 16) + (size_t)blockIdx.x * 4096;
@@ -575,7 +659,6 @@ __device__ __forceinline__ void k_ntt16_inv_low_body(u64 *__restrict__ lds, Batc
   // goes through LDS so that adjacent lanes read adjacent words (with mm,
   // of the product src x mul or src^2, formed here)
   if (mm) {
-    const ModQ M = mods[p];
     const u64 *mb = mm == 2 ? in
                             : batch_ptr(mul, blockIdx.y) + ((size_t)limb << 16) +
                                   (size_t)blockIdx.x * 4096;
@@ -583,7 +666,7 @@ __device__ __forceinline__ void k_ntt16_inv_low_body(u64 *__restrict__ lds, Batc
     for (int k = 0; k < 16; k++) {
       const int e = rl * 256 + c0 + 16 * k;
       const u64 v = in[e];
-      sm[lds16(rl, c0 + 16 * k)] = mul_mod(v, mm == 2 ? v : mb[e], M);
+      sm[lds16(rl, c0 + 16 * k)] = mul_lazy(v, mm == 2 ? v : mb[e], M);
     }
   } else {
 #pragma unroll
@@ -592,16 +675,9 @@ __device__ __forceinline__ void k_ntt16_inv_low_body(u64 *__restrict__ lds, Batc
   row_sync();
 #pragma unroll
   for (int j = 0; j < 16; j++) x[j] = sm[lds16(rl, 16 * c0 + j)];
-#pragma unroll
-  for (int b = 0; b < 4; b++) {
-    const int half = 1 << b;
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-      if (j & half) continue;
-      const int ti = (65536 >> (b + 1)) + ((row * 256 + 16 * c0 + j) >> (b + 1));
-      gs_bfly(x[j], x[j + half], W[ti], Ws[ti], q, q2);
-    }
-  }
+  u64_inv_round<3, false>(x, W, Ws, Q, [&](int b, int j) {
+    return (65536 >> (b + 1)) + ((row * 256 + 16 * c0 + j) >> (b + 1));
+  });
   row_sync();
 #pragma unroll
   for (int j = 0; j < 16; j++) sm[lds16(rl, 16 * c0 + j)] = x[j];
@@ -609,16 +685,10 @@ __device__ __forceinline__ void k_ntt16_inv_low_body(u64 *__restrict__ lds, Batc
   // round A^-1: column = c0 + 16 k, stages on column bits 4..7
 #pragma unroll
   for (int k = 0; k < 16; k++) x[k] = sm[lds16(rl, c0 + 16 * k)];
-#pragma unroll
-  for (int b = 4; b < 8; b++) {
-    const int half = 1 << (b - 4);
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-      if (k & half) continue;
-      const int ti = (65536 >> (b + 1)) + ((row * 256 + 16 * k) >> (b + 1));
-      gs_bfly(x[k], x[k + half], W[ti], Ws[ti], q, q2);
-    }
-  }
+  u64_inv_round<8, false>(x, W, Ws, Q, [&](int st, int k) {
+    const int b = 4 + st;
+    return (65536 >> (b + 1)) + ((row * 256 + 16 * k) >> (b + 1));
+  });
   // round Z^-1 (bits 8..11) on words t + 256 k: the thread's slots go back
   // (no other thread reads them), then each thread takes one tile column
 #pragma unroll
@@ -627,7 +697,7 @@ __device__ __forceinline__ void k_ntt16_inv_low_body(u64 *__restrict__ lds, Batc
   const int t = threadIdx.x;
 #pragma unroll
   for (int k = 0; k < 16; k++) x[k] = sm[lds16(k, t)];
-  u64_inv_round_z(x, W, Ws, blockIdx.x, q, q2);
+  u64_inv_round_z(x, W, Ws, blockIdx.x, Q);
 #pragma unroll
   for (int k = 0; k < 16; k++) out[t + 256 * k] = x[k];
 }
@@ -999,7 +1069,7 @@ __global__ __launch_bounds__(TPB) void k_ntt16m_fwd_high(Batch src, Batch dst, i
     u64 x[16];
 #pragma unroll
     for (int k = 0; k < 16; k++) x[k] = in[4096 * k];
-    u64_high_fwd(x, psi + ((size_t)p << 16), psi_sh + ((size_t)p << 16), qu, 2 * qu);
+    u64_high_fwd(x, psi + ((size_t)p << 16), psi_sh + ((size_t)p << 16), lazy_q(mods[p]));
 #pragma unroll
     for (int k = 0; k < 16; k++) out[4096 * k] = x[k];
   }
@@ -1055,7 +1125,7 @@ __global__ __launch_bounds__(TPB) void k_ntt16m_inv_high(
 #pragma unroll
     for (int k = 0; k < 16; k++) x[k] = io[4096 * k];
     u64_high_inv(x, ipsi + ((size_t)p << 16), ipsi_sh + ((size_t)p << 16), ninv[2 * p],
-                 ninv[2 * p + 1], qu, 2 * qu);
+                 ninv[2 * p + 1], lazy_q(mods[p]));
 #pragma unroll
     for (int k = 0; k < 16; k++) io[4096 * k] = x[k];
   }
@@ -1462,7 +1532,7 @@ __device__ __forceinline__ void low_key_64(u64 *__restrict__ sm, const LowKeyArg
                                            const u64 *__restrict__ psi,
                                            const u64 *__restrict__ psi_sh) {
   const ModQ M = mods[p];
-  const u64 q = M.q, q2 = 2 * q;
+  const LazyQ Q = lazy_q(M);
   const u64 *W = psi + ((size_t)p << 16);
   const u64 *Ws = psi_sh + ((size_t)p << 16);
   const int c0 = threadIdx.x & 15, rl = threadIdx.x >> 4;
@@ -1470,7 +1540,8 @@ __device__ __forceinline__ void low_key_64(u64 *__restrict__ sm, const LowKeyArg
   const u32 sb = (u32)(tile * 4096 + rl * 256 + 16 * c0);
   const u32 kslot = key_slot(sb);
   const int jo = l < a.q_limbs ? l / a.ds : -1;
-  // accumulators start at 0: add_mod(0, p) = p for the canonical products
+  // sums of at most kMaxDigits products below 2q: no carry, reduced once
+  static_assert(2 * kMaxDigits <= 16, "16q < 2^64");
   u64 acc0[16], acc1[16];
 #pragma unroll
   for (int i = 0; i < 16; i++) acc0[i] = acc1[i] = 0;
@@ -1485,7 +1556,7 @@ __device__ __forceinline__ void low_key_64(u64 *__restrict__ sm, const LowKeyArg
         load4(pa + i0, wa);
         if (a.own_mul == 1) load4(pb + i0, wb);
 #pragma unroll
-        for (int i = 0; i < 4; i++) y[i0 + i] = mul_mod(wa[i], a.own_mul == 2 ? wa[i] : wb[i], M);
+        for (int i = 0; i < 4; i++) y[i0 + i] = mul_lazy(wa[i], a.own_mul == 2 ? wa[i] : wb[i], M);
       }
     } else if (j == jo) {
       load16(batch_ptr(a.own, it) + ((size_t)l << 16) + sb, y);
@@ -1497,24 +1568,20 @@ __device__ __forceinline__ void low_key_64(u64 *__restrict__ sm, const LowKeyArg
       const int t = threadIdx.x;
 #pragma unroll
       for (int k = 0; k < 16; k++) y[k] = src[t + 256 * k];
-      u64_low_round_z(y, W, Ws, tile, q, q2);
+      u64_low_round_z(y, W, Ws, tile, Q);
       __syncthreads();
 #pragma unroll
       for (int k = 0; k < 16; k++) sm[lds16(k, t)] = y[k];
       __syncthreads();
 #pragma unroll
       for (int k = 0; k < 16; k++) y[k] = sm[lds16(rl, c0 + 16 * k)];
-      u64_low_round_a(y, W, Ws, row, q, q2);
+      u64_low_round_a(y, W, Ws, row, Q);
 #pragma unroll
       for (int k = 0; k < 16; k++) sm[lds16(rl, c0 + 16 * k)] = y[k];
       row_sync();
 #pragma unroll
       for (int i = 0; i < 16; i++) y[i] = sm[lds16(rl, 16 * c0 + i)];
-      u64_low_round_b(y, W, Ws, row, c0, q, q2);
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        y[i] = csub(csub(y[i], q2), q);
-      }
+      u64_low_round_b(y, W, Ws, row, c0, Q);
     }
     const u64 *kb = a.key + ((size_t)(2 * j) * a.K + p) * 65536 + kslot;
     const u64 *ka = kb + (size_t)a.K * 65536;
@@ -1540,18 +1607,17 @@ __device__ __forceinline__ void low_key_64(u64 *__restrict__ sm, const LowKeyArg
       for (int i = 0; i < 4; i++) {
         const int e = 4 * g + i;
         const u64 b = kw[g & 1][2 * i], c = kw[g & 1][2 * i + 1];
-        const u64 pb = redc(__umul64hi(y[e], b), y[e] * b, q, M.qinv);
-        const u64 pa = redc(__umul64hi(y[e], c), y[e] * c, q, M.qinv);
-        acc0[e] = add_mod(acc0[e], pb, q);
-        acc1[e] = add_mod(acc1[e], pa, q);
+        // y lazy (any word), the key word below q
+        acc0[e] += redc_lazy(__umul64hi(y[e], b), y[e] * b, Q.q, M.qinv);
+        acc1[e] += redc_lazy(__umul64hi(y[e], c), y[e] * c, Q.q, M.qinv);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
   u64 *o = a.acc + it * a.acc_stride + ((size_t)l << 16);
   const u32 tb = a.ginv == 1 ? sb & ~4095u : autom_index(sb, a.ginv, 16) & ~4095u;
-  low_key_store(sm, [&](int i) { return acc0[i]; }, sb, a.ginv, o, tb);
-  low_key_store(sm, [&](int i) { return acc1[i]; }, sb, a.ginv, o + ((size_t)a.E << 16), tb);
+  low_key_store(sm, [&](int i) { return lazy_canon(acc0[i], Q); }, sb, a.ginv, o, tb);
+  low_key_store(sm, [&](int i) { return lazy_canon(acc1[i], Q); }, sb, a.ginv, o + ((size_t)a.E << 16), tb);
 }
 
 // One kernel per body, each over a run of nl limbs of its kind starting at
@@ -2689,8 +2755,8 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
   }
   // the high passes' 15 twiddles of every target's prime (forward) and every
   // source's prime (inverse), 32 words each: fp64 primes as 16 (w, w / q)
-  // pairs, others as [16] psi_br and [16] Shoup constants; entry 0 is unused
-  // and word 0 holds q.  Each lane group works on its own primes, so these
+  // pairs, others as [16] psi_br and [16] Shoup constants; entry 0 is unused:
+  // word 0 holds q, word 16 floor(2^64 / q) of the others.  Each lane group works on its own primes, so these
   // would otherwise be per-lane global loads.
   u64 *ttw = tgt + (size_t)nd * TW, *stw = ttw + (size_t)nd * 32;
   // RS: the lifts, [RSD][16 rows][64 columns of the block]
@@ -2709,6 +2775,7 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
     const u64 qu = mods[pt].q;
     if (j == 0) {
       w[0] = qu;
+      if (qu >= kFpPrimeBound) w[16] = lazy_q(mods[pt]).mu;
       continue;
     }
     const size_t o = ((size_t)pt << 16) + j;
@@ -2760,7 +2827,8 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
         // before the kernel (with the x N^-1, x canonical)
         u64 hw = tab[4 * ns + s], hws = tab[5 * ns + s];
         if (!wide_src_out) {
-          u64_high_inv_stages(x, sw0, sw0 + 16, qu, 2 * qu);
+          LazyQ Q{qu, 0 - qu, (u32)sw0[16], 0, 0};
+          u64_high_inv_stages(x, sw0, sw0 + 16, Q);
           hw = tab[s];
           hws = tab[ns + s];
         }
@@ -2967,7 +3035,8 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
         // stored canonical for the launch after the kernel
         if (!wide_tgt_out) {
           const u64 qu = w[0];
-          u64_high_fwd(y[ee], tw0, tw0 + 16, qu, 2 * qu);
+          LazyQ Q{qu, 0 - qu, (u32)tw0[16], 0, 0};
+          u64_high_fwd(y[ee], tw0, tw0 + 16, Q);
         }
 #pragma unroll
         for (int r = 0; r < 16; r++) po[4096 * r] = y[ee][r];

@@ -887,3 +887,33 @@ def test_align_to_changes_the_scale():
     assert fhe.align_to(ct, near, ctx) is ct
     with pytest.raises(ValueError):
         fhe.align_to(ct, ct.state.replace(scaling_factor=ct.state.scaling_factor * 1.5), ctx)
+
+
+@pytest.mark.parametrize("first_mod,dcrt_bits,special_bits", [(46, 46, 47), (53, 50, 59), (60, 59, 60)])
+@pytest.mark.parametrize("fill", ["max", "alternate", "one_max"])
+def test_ntt_lazy_bounds_full_size(fill, first_mod, dcrt_bits, special_bits):
+    """The 64-bit transforms at N = 2^16 over their range of primes (46 to 60
+    bits), on words that drive the unreduced sums to their ends: every word
+    q - 1, q - 1 and 0 in turn, one non-zero word."""
+    from easyfhe import _native
+
+    p = dict(log_n=16, depth=3, dnum=2, dcrt_bits=dcrt_bits, first_mod=first_mod,
+             special_bits=special_bits)
+    client, ctx = device_context(p, relin=False)
+    orc = oracle_context(p)
+    L, A, N = orc.L, orc.alpha, orc.N
+    a = np.zeros((1, L + A, N), dtype=np.uint64)
+    for l in range(L + A):
+        top = np.uint64(int(orc.primes[l]) - 1)
+        if fill == "max":
+            a[0, l] = top
+        elif fill == "alternate":
+            a[0, l, ::2] = top
+        else:
+            a[0, l, 4097 * (l + 1)] = top
+    for inverse, exp in ((0, orc.ntt_limbs(a[0], q_limbs=L)), (1, orc.intt_limbs(a[0], q_limbs=L))):
+        got = np.zeros_like(a)
+        _native.check(_native.lib.ckks_poly_ntt(ctx.handle, a.ctypes.data_as(_native.U64P),
+                                                got.ctypes.data_as(_native.U64P), 1, L + A, L,
+                                                inverse))
+        assert np.array_equal(got[0], exp), inverse
