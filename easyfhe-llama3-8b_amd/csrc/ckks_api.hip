@@ -1073,6 +1073,14 @@ static bool ks_modup(ckks_context *c, int limbs, int n, const u64 *const *d, u64
     }
     return packed;
   }
+  if (!high_only && ring_convert_ok(c, std::min(c->ds, limbs))) {
+    const BCTable *tabs[kMaxDigits];
+    for (int j = 0; j < digits; j++) tabs[j] = &bc_up(c, limbs, j);
+    launch_ring_sources(c, src, strided(coeff, (size_t)limbs * N), n, 0, limbs, limbs, tabs, c->ds);
+    launch_ring_modup(c, Strided{coeff, (u64)limbs * N}, Strided{ext, (u64)digits * E * N}, src,
+                      own_copy, n, limbs, digits, tabs);
+    return false;
+  }
   launch_ntt(c, src, strided(coeff, (size_t)limbs * N), n, 0, limbs, limbs, true);
   for (int j = 0; j < digits; j++) {
     const int lo = j * c->ds, hi = std::min((j + 1) * c->ds, limbs), ns = hi - lo;
@@ -1100,6 +1108,7 @@ struct KsJob {
   u64 galois;
   const u64 *add0, *add1;
   u64 *out0, *out1;
+  const u64 *plus = nullptr;  // [2][limbs][N] added as it is (ring_convert_ok(alpha) only)
 };
 
 // The key product of the fp64 Q limbs left by ks_modup_inner for ks_moddown
@@ -1141,6 +1150,24 @@ static void ks_moddown(ckks_context *c, int limbs, u64 *acc, const std::vector<K
     uniform = (jobs[i].add1 ? (u64)(jobs[i].add1 - jobs[i].add0) : 0) == add1_off &&
               (!jobs[i].add1 || jobs[i].add0) && (u64)(jobs[i].out1 - jobs[i].out0) == out1_off;
   const Batch spb = strided(ptmp - (size_t)limbs * N, (size_t)c->alpha * N);  // limb l at l N
+  if (ring_convert_ok(c, c->alpha)) {
+    const BCTable &down = bc_down(c, limbs), *dp = &down;
+    launch_ring_sources(c, strided(acc, E * N), spb, 2 * n, limbs, c->alpha, limbs, &dp, c->alpha);
+    for (int b0 = 0; b0 < n; b0 += kMaxBatch) {
+      const int nb = std::min(kMaxBatch, n - b0);
+      RingItem items[kMaxBatch];
+      for (int i = 0; i < nb; i++) {
+        const KsJob &jb = jobs[b0 + i];
+        items[i] = RingItem{jb.add0, jb.add1, jb.plus, jb.out0, jb.out1, jb.galois};
+      }
+      launch_ring_moddown(c, Strided{ptmp + (size_t)b0 * 2 * c->alpha * N, (u64)c->alpha * N},
+                          Strided{acc + (size_t)b0 * 2 * E * N, (u64)2 * E * N}, items, nb, limbs,
+                          pinv, down);
+    }
+    return;
+  }
+  for (const KsJob &jb : jobs)
+    if (jb.plus) throw std::logic_error("ModDown: added ciphertexts on the ring path only");
   u64 *conv = s.get((size_t)n * 2 * limbs * N);
   // N = 2^16: the special limbs' inverse high pass, the conversion and the
   // forward high pass of the Q limbs in one kernel, then the low pass with
@@ -1221,12 +1248,22 @@ static u64 *ks_inner(ckks_context *c, int limbs, const u64 *ext, const std::vect
     launch_key_inner(c, strided((u64 *)ext, est), strided(acc, 2 * E * N), n, *jobs[0].key,
                      digits, E, limbs, jobs[0].galois, own ? &ob : nullptr);
   } else {
-    for (int i = 0; i < n; i++) {
+    for (int b0 = 0; b0 < n; b0 += kMaxBatch) {
+      const int nb = std::min(kMaxBatch, n - b0);
+      int items[kMaxBatch];
+      const DeviceKey *keys[kMaxBatch];
+      u64 gal[kMaxBatch];
       Batch ob{};
-      if (own) ob.p[0] = (u64 *)own[jobs[i].ext_item];
-      launch_key_inner(c, strided((u64 *)ext + (size_t)jobs[i].ext_item * est, 0),
-                       strided(acc + (size_t)i * 2 * E * N, 0), 1, *jobs[i].key, digits, E,
-                       limbs, jobs[i].galois, own ? &ob : nullptr);
+      for (int i = 0; i < nb; i++) {
+        const KsJob &jb = jobs[b0 + i];
+        items[i] = jb.ext_item;
+        keys[i] = jb.key;
+        gal[i] = jb.galois;
+        if (own) ob.p[jb.ext_item] = (u64 *)own[jb.ext_item];
+      }
+      launch_key_inner_jobs(c, Strided{(u64 *)ext, (u64)est},
+                            Strided{acc + (size_t)b0 * 2 * E * N, (u64)2 * E * N}, nb, items, keys,
+                            gal, digits, E, limbs, own ? &ob : nullptr);
     }
   }
   return acc;
@@ -2658,6 +2695,39 @@ int ckks_hoisted_mac_sum(ckks_context *c, const ckks_ct *const *babies, int B,
   for (int b = 0; b < B; b++) bb.p[b] = babies[b]->d;
   ckks_ct *acc = nullptr;
   Scratch s(c);
+  if (giant_count > 1 && gg != 1 && ring_convert_ok(c, c->alpha)) {
+    // a small ring: the groups' MACs in few launches, then one key switch a
+    // group whose ModDown adds the group's MAC
+    const DeviceKey &key = get_key(c, gg);
+    const int per = std::max(1, kMacGroupPts / B), chunk = std::min(giant_count, 64);
+    u64 *inner = s.get((size_t)chunk * 2 * P), *turn[2] = {s.get(2 * P), s.get(2 * P)};
+    std::vector<const u64 *> pt((size_t)B * giant_count);
+    for (size_t i = 0; i < pt.size(); i++) pt[i] = pts[i]->d;
+    acc = new_ct(c, 2, limbs, 0, babies[0]->slots, scale, sdeg);
+    const u64 *cur = nullptr;
+    for (int g1 = giant_count; g1 > 0; g1 -= chunk) {
+      const int g0 = std::max(0, g1 - chunk);
+      for (int g = g0; g < g1; g += per)
+        launch_mac_groups(c, bb, pt.data() + (size_t)g * B, B, std::min(per, g1 - g),
+                          inner + (size_t)(g - g0) * 2 * P, limbs);
+      for (int g = g1 - 1; g >= g0; g--) {
+        const u64 *in = inner + (size_t)(g - g0) * 2 * P;
+        if (!cur) {
+          cur = in;
+          continue;
+        }
+        u64 *dst = g == 0 ? acc->d : turn[g & 1];
+        const u64 *d = cur + P;
+        Scratch s2(c);
+        std::vector<KsJob> job{KsJob{0, &key, gg, cur, nullptr, dst, dst + P, in}};
+        u64 *ka = ks_modup_inner(c, limbs, 1, &d, job, s2);
+        ks_moddown(c, limbs, ka, job, s2);
+        cur = dst;
+      }
+    }
+    *out = acc;
+    return CKKS_OK;
+  }
   u64 *inner = s.get(2 * P);
   for (int g = giant_count - 1; g >= 0; g--) {
     Batch bp{};

@@ -33,6 +33,11 @@ constexpr int kMacCtsFp = 8;        // the same for its fp64 path
 constexpr int kTabGroups = 16;      // giant groups of one Q-basis MAC pass (k_mac_table)
 constexpr int kTabCts = 2;          // ciphertexts per plaintext read in that pass
 constexpr int kTabCtsFp = 8;        // the same for its fp64 path
+constexpr int kMacGroupPts = 256;   // plaintexts of one launch_mac_groups
+// Source primes of a conversion inside a ring kernel: each target's block
+// forms its own sums, about 20 instructions a source and word, against 100 a
+// word for the transform; beyond 4 the separate conversion shares more
+constexpr int kRingSources = 4;
 constexpr int kMultiItems = 4;    // items per multi-rotation key inner product launch
 
 // Per-prime constants, resident in device memory.
@@ -46,11 +51,13 @@ struct ModQ {
 };
 
 // A set of polynomials addressed either by explicit pointers (p[i]) or by a
-// base and a stride (base + i * stride) when base != nullptr.
+// base and a stride (base + i * stride) when base != nullptr.  Kernel
+// arguments are read from host memory: base, stride and the first pointers
+// share a line.
 struct Batch {
-  u64 *p[kMaxBatch];
   u64 *base;
   u64 stride;
+  u64 *p[kMaxBatch];
 };
 
 // An internal buffer of equally spaced items.
@@ -71,8 +78,11 @@ struct PostOp {
   const u64 *scal;
 };
 
+// (both forms are read before the choice, so that a block waits for its
+// arguments once; an index past the pointers is one of a strided batch)
 __device__ __forceinline__ u64 *batch_ptr(const Batch &b, int i) {
-  return b.base ? b.base + (u64)i * b.stride : b.p[i];
+  u64 *p = b.p[i & (kMaxBatch - 1)];
+  return b.base ? b.base + (u64)i * b.stride : p;
 }
 
 // item i of a batch on the host (null for an empty batch's item 0)
@@ -472,6 +482,38 @@ void launch_copy_limbs(ckks_context *c, const Batch &src, const Batch &dst, int 
 void launch_key_inner(ckks_context *c, const Batch &ext, const Batch &acc, int n_items,
                       const DeviceKey &key, int digits, int E, int q_limbs, u64 galois,
                       const Batch *own = nullptr);
+// launch_key_inner of up to 64 jobs, each with an extended item (ext item
+// items[i]), a key and an automorphism of its own: acc item i
+void launch_key_inner_jobs(ckks_context *c, const Strided &ext, const Strided &acc, int n_jobs,
+                           const int *items, const DeviceKey *const *keys, const u64 *galois,
+                           int digits, int E, int q_limbs, const Batch *own);
+// N = 2^10 .. 2^14: whether a conversion from ns primes runs inside the
+// whole-ring kernels below
+bool ring_convert_ok(const ckks_context *c, int ns);
+// the inverse NTT of limbs that the conversions below read, each times its
+// source constant [Qhat^-1]_q of tabs[i / per], source i % per (limb l_begin + i)
+void launch_ring_sources(ckks_context *c, const Batch &src, const Batch &dst, int n_items,
+                         int l_begin, int l_count, int q_limbs, const BCTable *const *tabs,
+                         int per);
+// every digit's conversion and forward NTT: coeff per item [limbs][N] from
+// launch_ring_sources, ext per item [digits][E][N], tabs the digits'
+// conversion tables; own limbs copied from own with own_copy
+void launch_ring_modup(ckks_context *c, const Strided &coeff, const Strided &ext, const Batch &own,
+                       bool own_copy, int n_items, int limbs, int digits,
+                       const BCTable *const *tabs);
+// An item of the ring ModDown: its pointers and automorphism share one line of
+// the kernel's arguments, which are read from host memory (as five Batch
+// arguments, read one after the other, they cost 2 us a launch).
+struct RingItem {
+  const u64 *add0, *add1, *plus;  // plus: [2][limbs][N] (each null: none)
+  u64 *out0, *out1;
+  u64 galois;
+};
+// the ModDown's conversion (sp: per item and component the special limbs from
+// launch_ring_sources), forward NTT and combine
+void launch_ring_moddown(ckks_context *c, const Strided &sp, const Strided &acc,
+                         const RingItem *items, int n_items, int limbs, const u64 *pinv,
+                         const BCTable &tab);
 // N = 2^16: the high pass of the forward NTT alone (the low pass then runs in
 // launch_ntt_low_key)
 void launch_ntt_fwd_high(ckks_context *c, const Batch &src, const Batch &dst, int n_items,
@@ -607,6 +649,10 @@ void launch_ext_rot_accum(ckks_context *c, const Batch &u, const Batch &acc, con
 // limbs (an extended object: Q limbs then alpha P limbs)
 void launch_mac(ckks_context *c, const Batch &babies, const Batch &pts, int B, u64 *out,
                 int limbs_total, int q_limbs);
+// the Q-basis MACs of G groups sharing the babies, out [G][2][limbs][N]
+// (B G <= kMacGroupPts)
+void launch_mac_groups(ckks_context *c, const Batch &babies, const u64 *const *pts, int B, int G,
+                       u64 *out, int limbs);
 void launch_keygen(ckks_context *c, DeviceKey &key, u64 id, int relin, u64 galois);
 // residues of a signed integer polynomial e[N] over `limbs` limbs, then NTT
 void launch_expand_ntt(ckks_context *c, const long long *e, u64 *out, int limbs, int q_limbs);

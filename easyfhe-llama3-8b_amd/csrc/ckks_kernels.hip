@@ -1168,6 +1168,552 @@ static void ntt16_dispatch(ckks_context *c, const Batch &src, const Batch &dst, 
   }
 }
 
+// ===========================================================================
+// Rings of N = 2^10 .. 2^14: a block holds one whole limb-polynomial, 2^LW
+// words a thread in registers, and exchanges it through LDS between rounds of
+// LW stages, so a transform is one launch and one pass over memory, and the
+// conversion of a key switch's ModUp or ModDown before it and the combine
+// after it run in the same block.
+//
+// A call on one ciphertext of such a ring has 4 to 20 limb-polynomials: fewer
+// than the chip has CUs, so it takes as long as its chain of launches, and a
+// launch as long as one block's chain of loads, stages and exchanges.  The
+// two-pass radix-2 kernels this replaced exchanged after every stage (13
+// barriers, 26 us a transform of N = 2^13 in two launches, now 10.5 us for
+// fp64 primes and 12.5 us for 60-bit ones; about half of it VALU issue on the
+// block's one CU, half waits).  A key switch of 4 + 1 limbs is 5 launches
+// (350 -> 58 us), the 128 x 128 product 2792 -> 537 us.
+// Word positions: in the window at bit lo, word k of thread t is position
+//   (t >> lo) << (lo + LW) | k << lo | (t & (2^lo - 1)),
+// so a round's stages are on bits of k.  A thread writes back the LDS words
+// that it read, so an exchange needs one barrier; the next round's twiddles
+// are loaded ahead of it.
+// ===========================================================================
+template <int LOGN, int LW>
+struct Ring {
+  static constexpr int N = 1 << LOGN, W = 1 << LW, T = N >> LW;
+  static constexpr int R = (LOGN + LW - 1) / LW;  // rounds
+  static constexpr int kLds = N + (N >> 4);       // one word of padding in 16
+  // forward round i: stages on bits [flo(i), fhi(i)), high to low, window at flo(i)
+  static constexpr int fhi(int i) { return LOGN - i * LW; }
+  static constexpr int flo(int i) { return fhi(i) > LW ? fhi(i) - LW : 0; }
+  // inverse round i: stages on bits [ilo(i), ihi(i)), low to high, window at iwin(i)
+  static constexpr int ilo(int i) { return i * LW; }
+  static constexpr int ihi(int i) { return ilo(i) + LW < LOGN ? ilo(i) + LW : LOGN; }
+  static constexpr int iwin(int i) { return ihi(i) - LW; }
+  static __device__ __forceinline__ int pos(int lo, int k, int t) {
+    return ((t >> lo) << (lo + LW)) | (k << lo) | (t & ((1 << lo) - 1));
+  }
+  static __device__ __forceinline__ int slot(int j) { return j + (j >> 4); }
+};
+
+// the next round's twiddles before a round's butterflies (8 words a thread) or
+// after them (16 words: two sets of 15 do not fit 128 registers)
+template <int LW>
+constexpr bool kEarly = LW <= 3;
+
+// Twiddles of a window's stages: entry m of the stage on bit i of k (its
+// pairs with k >> (i + 1) = m) at index 2^(LW - 1 - i) - 1 + m.
+template <int LW>
+struct Tw64 {
+  u64 w[1 << LW], ws[1 << LW];
+};
+template <int LW>
+struct TwFp {
+  double2 w[1 << LW];
+};
+
+// stages on bits [lo, hi) of a window at win
+template <int LOGN, int LW>
+__device__ __forceinline__ void ring_tw(Tw64<LW> &tw, const u64 *__restrict__ W,
+                                        const u64 *__restrict__ Ws, int win, int lo, int hi,
+                                        int t) {
+#pragma unroll
+  for (int i = LW - 1; i >= 0; i--) {
+    if (win + i < lo || win + i >= hi) continue;
+#pragma unroll
+    for (int m = 0; m < (1 << (LW - 1 - i)); m++) {
+      const int o = (1 << (LOGN - 1 - win - i)) + (((t >> win) << (LW - 1 - i)) | m);
+      tw.w[(1 << (LW - 1 - i)) - 1 + m] = W[o];
+      tw.ws[(1 << (LW - 1 - i)) - 1 + m] = Ws[o];
+    }
+  }
+}
+template <int LOGN, int LW>
+__device__ __forceinline__ void ring_tw(TwFp<LW> &tw, const double2 *__restrict__ W,
+                                        const double2 *, int win, int lo, int hi, int t) {
+#pragma unroll
+  for (int i = LW - 1; i >= 0; i--) {
+    if (win + i < lo || win + i >= hi) continue;
+#pragma unroll
+    for (int m = 0; m < (1 << (LW - 1 - i)); m++)
+      tw.w[(1 << (LW - 1 - i)) - 1 + m] =
+          W[(1 << (LOGN - 1 - win - i)) + (((t >> win) << (LW - 1 - i)) | m)];
+  }
+}
+
+template <int LOGN, int LW, typename X>
+__device__ __forceinline__ void ring_exchange(X (&x)[1 << LW], X *__restrict__ sm, int from,
+                                              int to, int t) {
+  using G = Ring<LOGN, LW>;
+#pragma unroll
+  for (int k = 0; k < G::W; k++) sm[G::slot(G::pos(from, k, t))] = x[k];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < G::W; k++) x[k] = sm[G::slot(G::pos(to, k, t))];
+}
+
+// Forward rounds RI .. R - 1 of words in the window flo(RI), tw their first
+// round's twiddles.  64-bit: words enter below q; stages 3, 6, 9, 12 reduce
+// their X operands (bounds in units of q: 5, 9, 13, R 6+, 10+, 14+, R 6+ ...;
+// ct_bfly takes X < 12q without a reduction); the result is any word.
+template <int LOGN, int LW, int RI>
+__device__ __forceinline__ void ring_fwd(u64 (&x)[1 << LW], Tw64<LW> &tw, u64 *__restrict__ sm,
+                                         const u64 *__restrict__ W, const u64 *__restrict__ Ws,
+                                         const LazyQ &Q, int t) {
+  using G = Ring<LOGN, LW>;
+  constexpr int lo = G::flo(RI), hi = G::fhi(RI);
+  Tw64<LW> nx;
+  if constexpr (kEarly<LW> && RI + 1 < G::R)
+    ring_tw<LOGN, LW>(nx, W, Ws, G::flo(RI + 1), G::flo(RI + 1), G::fhi(RI + 1), t);
+#pragma unroll
+  for (int i = LW - 1; i >= 0; i--) {
+    if (lo + i >= hi) continue;
+    const int st = LOGN - 1 - lo - i, half = 1 << i;
+    const bool red = st >= 3 && st % 3 == 0;
+#pragma unroll
+    for (int k = 0; k < G::W; k++) {
+      if (k & half) continue;
+      const int s = (1 << (LW - 1 - i)) - 1 + (k >> (i + 1));
+      if (red) ct_bfly<true>(x[k], x[k + half], tw.w[s], tw.ws[s], Q);
+      else ct_bfly<false>(x[k], x[k + half], tw.w[s], tw.ws[s], Q);
+    }
+  }
+  if constexpr (RI + 1 < G::R) {
+    if constexpr (!kEarly<LW>)
+      ring_tw<LOGN, LW>(nx, W, Ws, G::flo(RI + 1), G::flo(RI + 1), G::fhi(RI + 1), t);
+    ring_exchange<LOGN, LW>(x, sm, lo, G::flo(RI + 1), t);
+    ring_fwd<LOGN, LW, RI + 1>(x, nx, sm, W, Ws, Q, t);
+  }
+}
+
+// fp64: |x| grows by at most q a stage from |x| < q, below 15q < 2^49
+template <int LOGN, int LW, int RI>
+__device__ __forceinline__ void ring_fwd(double (&x)[1 << LW], TwFp<LW> &tw,
+                                         double *__restrict__ sm, const double2 *__restrict__ W,
+                                         double q, int t) {
+  using G = Ring<LOGN, LW>;
+  constexpr int lo = G::flo(RI), hi = G::fhi(RI);
+  TwFp<LW> nx;
+  if constexpr (kEarly<LW> && RI + 1 < G::R)
+    ring_tw<LOGN, LW>(nx, W, W, G::flo(RI + 1), G::flo(RI + 1), G::fhi(RI + 1), t);
+#pragma unroll
+  for (int i = LW - 1; i >= 0; i--) {
+    if (lo + i >= hi) continue;
+    const int half = 1 << i;
+#pragma unroll
+    for (int k = 0; k < G::W; k++) {
+      if (k & half) continue;
+      const double2 w = tw.w[(1 << (LW - 1 - i)) - 1 + (k >> (i + 1))];
+      ct_fp(x[k], x[k + half], w.x, w.y, q);
+    }
+  }
+  if constexpr (RI + 1 < G::R) {
+    if constexpr (!kEarly<LW>)
+      ring_tw<LOGN, LW>(nx, W, W, G::flo(RI + 1), G::flo(RI + 1), G::fhi(RI + 1), t);
+    ring_exchange<LOGN, LW>(x, sm, lo, G::flo(RI + 1), t);
+    ring_fwd<LOGN, LW, RI + 1>(x, nx, sm, W, q, t);
+  }
+}
+
+// inv_plan for the stages on bits [s0, s1) of k of a 2^LW-word round
+template <int LW>
+struct RingInvPlan {
+  bool red[LW + 1][1 << LW];
+};
+template <int LW>
+constexpr RingInvPlan<LW> ring_inv_plan(int in, int s0, int s1, bool last) {
+  RingInvPlan<LW> p{};
+  int b[1 << LW] = {};
+  for (int k = 0; k < 1 << LW; k++) b[k] = in;
+  for (int st = s0; st < s1; st++) {
+    const int half = 1 << st;
+    for (int k = 0; k < 1 << LW; k++) {
+      p.red[st][k] = b[k] > 8;
+      if (b[k] > 8) b[k] = 3;
+    }
+    for (int k = 0; k < 1 << LW; k++) {
+      if (k & half) continue;
+      b[k] = b[k] + b[k + half];
+      b[k + half] = 4;
+    }
+  }
+  for (int k = 0; k < 1 << LW; k++) p.red[LW][k] = !last && b[k] > 8;
+  return p;
+}
+
+// Inverse rounds RI .. R - 1 of words in the window iwin(RI), canonical on
+// entry to round 0; any word after the last round (64-bit), |x| <= 16q (fp64)
+template <int LOGN, int LW, int RI>
+__device__ __forceinline__ void ring_inv(u64 (&x)[1 << LW], Tw64<LW> &tw, u64 *__restrict__ sm,
+                                         const u64 *__restrict__ W, const u64 *__restrict__ Ws,
+                                         const LazyQ &Q, int t) {
+  using G = Ring<LOGN, LW>;
+  constexpr int win = G::iwin(RI), s0 = G::ilo(RI) - win, s1 = G::ihi(RI) - win;
+  constexpr RingInvPlan<LW> plan = ring_inv_plan<LW>(RI ? 8 : 1, s0, s1, RI + 1 == G::R);
+  Tw64<LW> nx;
+  if constexpr (kEarly<LW> && RI + 1 < G::R)
+    ring_tw<LOGN, LW>(nx, W, Ws, G::iwin(RI + 1), G::ilo(RI + 1), G::ihi(RI + 1), t);
+#pragma unroll
+  for (int i = s0; i < s1; i++) {
+    const int half = 1 << i;
+#pragma unroll
+    for (int k = 0; k < G::W; k++)
+      if (plan.red[i][k]) x[k] = lazy_reduce(x[k], Q);
+#pragma unroll
+    for (int k = 0; k < G::W; k++) {
+      if (k & half) continue;
+      const int s = (1 << (LW - 1 - i)) - 1 + (k >> (i + 1));
+      gs_bfly(x[k], x[k + half], tw.w[s], tw.ws[s], Q);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < G::W; k++)
+    if (plan.red[LW][k]) x[k] = lazy_reduce(x[k], Q);
+  if constexpr (RI + 1 < G::R) {
+    if constexpr (!kEarly<LW>)
+      ring_tw<LOGN, LW>(nx, W, Ws, G::iwin(RI + 1), G::ilo(RI + 1), G::ihi(RI + 1), t);
+    ring_exchange<LOGN, LW>(x, sm, win, G::iwin(RI + 1), t);
+    ring_inv<LOGN, LW, RI + 1>(x, nx, sm, W, Ws, Q, t);
+  }
+}
+
+template <int LOGN, int LW, int RI>
+__device__ __forceinline__ void ring_inv(double (&x)[1 << LW], TwFp<LW> &tw,
+                                         double *__restrict__ sm, const double2 *__restrict__ W,
+                                         double q, double qinv, int t) {
+  using G = Ring<LOGN, LW>;
+  constexpr int win = G::iwin(RI), s0 = G::ilo(RI) - win, s1 = G::ihi(RI) - win;
+  TwFp<LW> nx;
+  if constexpr (kEarly<LW> && RI + 1 < G::R)
+    ring_tw<LOGN, LW>(nx, W, W, G::iwin(RI + 1), G::ilo(RI + 1), G::ihi(RI + 1), t);
+  if constexpr (RI > 0) {
+#pragma unroll
+    for (int k = 0; k < G::W; k++) x[k] = fp_reduce(x[k], qinv, q);
+  }
+#pragma unroll
+  for (int i = s0; i < s1; i++) {
+    const int half = 1 << i;
+#pragma unroll
+    for (int k = 0; k < G::W; k++) {
+      if (k & half) continue;
+      const double2 w = tw.w[(1 << (LW - 1 - i)) - 1 + (k >> (i + 1))];
+      gs_fp(x[k], x[k + half], w.x, w.y, q);
+    }
+  }
+  if constexpr (RI + 1 < G::R) {
+    if constexpr (!kEarly<LW>)
+      ring_tw<LOGN, LW>(nx, W, W, G::iwin(RI + 1), G::ilo(RI + 1), G::ihi(RI + 1), t);
+    ring_exchange<LOGN, LW>(x, sm, win, G::iwin(RI + 1), t);
+    ring_inv<LOGN, LW, RI + 1>(x, nx, sm, W, q, qinv, t);
+  }
+}
+
+struct RingTabs {
+  const ModQ *mods;
+  const u64 *psi, *psi_sh;
+  const double2 *tw;  // fp64 (w, w / q), primes below 2^45
+  const u64 *ninv;    // inverse: [K][2] N^-1 and its Shoup constant
+  const double2 *ninv_fp;
+};
+
+// Forward transform of canonical words x (window at flo(0)) of prime p:
+// canonical words of positions t + T k (the last exchange brings the words
+// into the order in which a wave's loads and stores are contiguous)
+template <int LOGN, int LW>
+__device__ __forceinline__ void ring_forward(u64 (&x)[1 << LW], u64 *__restrict__ lds,
+                                             const RingTabs &rt, int p, int t) {
+  using G = Ring<LOGN, LW>;
+  const ModQ M = rt.mods[p];
+  if (M.q < kFpPrimeBound) {
+    const double q = (double)M.q, qinv = 1.0 / q;
+    const double2 *W = rt.tw + ((size_t)p << LOGN);
+    TwFp<LW> tw;
+    ring_tw<LOGN, LW>(tw, W, W, G::flo(0), G::flo(0), G::fhi(0), t);
+    double xd[G::W];
+#pragma unroll
+    for (int k = 0; k < G::W; k++) xd[k] = u52_to_dbl(x[k]);
+    ring_fwd<LOGN, LW, 0>(xd, tw, reinterpret_cast<double *>(lds), W, q, t);
+#pragma unroll
+    for (int k = 0; k < G::W; k++) x[k] = fp_canon(xd[k], qinv, q);
+  } else {
+    const LazyQ Q = lazy_q(M);
+    const u64 *W = rt.psi + ((size_t)p << LOGN), *Ws = rt.psi_sh + ((size_t)p << LOGN);
+    Tw64<LW> tw;
+    ring_tw<LOGN, LW>(tw, W, Ws, G::flo(0), G::flo(0), G::fhi(0), t);
+    ring_fwd<LOGN, LW, 0>(x, tw, lds, W, Ws, Q, t);
+#pragma unroll
+    for (int k = 0; k < G::W; k++) x[k] = lazy_canon(x[k], Q);
+  }
+  ring_exchange<LOGN, LW>(x, lds, 0, LOGN - LW, t);
+}
+
+// Tables of a key switch's digits (or of the special limbs; per 0: none): limb
+// l_begin + i is source i % per of tab[i / per], whose digit has
+// min(per, limbs - i / per per) sources
+struct RingDigits {
+  const u64 *tab[kMaxDigits];
+  int per, limbs;
+};
+
+// Transforms of limbs l_begin + blockIdx.x of items blockIdx.y.  INV with
+// tables (BCTable::sn): the words leave as [x N^-1 Qhat^-1]_q, the first
+// product of the conversion that reads them.
+template <int LOGN, int LW, bool INV>
+__global__ __launch_bounds__((1 << (LOGN - LW))) void k_ring_ntt(Batch src, Batch dst,
+                                                                 int l_begin, int q_limbs, int L,
+                                                                 RingTabs rt, RingDigits dg) {
+  using G = Ring<LOGN, LW>;
+  __shared__ u64 lds[G::kLds];
+  const int t = threadIdx.x, limb = l_begin + blockIdx.x;
+  const int p = prime_of(limb, q_limbs, L);
+  const u64 *in = batch_ptr(src, blockIdx.y) + ((size_t)limb << LOGN);
+  u64 *out = batch_ptr(dst, blockIdx.y) + ((size_t)limb << LOGN);
+  u64 x[G::W];
+  if constexpr (!INV) {
+#pragma unroll
+    for (int k = 0; k < G::W; k++) x[k] = in[G::pos(G::flo(0), k, t)];
+    ring_forward<LOGN, LW>(x, lds, rt, p, t);
+#pragma unroll
+    for (int k = 0; k < G::W; k++) out[t + G::T * k] = x[k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < G::W; k++) x[k] = in[t + G::T * k];
+    ring_exchange<LOGN, LW>(x, lds, LOGN - LW, 0, t);
+    const ModQ M = rt.mods[p];
+    const u64 *sn = nullptr;
+    int sns = 0, si = 0;
+    if (dg.per) {
+      const int i = blockIdx.x, lo = i / dg.per * dg.per;
+      sn = dg.tab[i / dg.per];
+      sns = min(dg.per, dg.limbs - lo);
+      si = i - lo;
+    }
+    if (M.q < kFpPrimeBound) {
+      const double q = (double)M.q, qinv = 1.0 / q;
+      const double2 *W = rt.tw + ((size_t)p << LOGN);
+      const double2 ni = sn ? reinterpret_cast<const double2 *>(sn + 2 * sns)[si] : rt.ninv_fp[p];
+      TwFp<LW> tw;
+      ring_tw<LOGN, LW>(tw, W, W, G::iwin(0), G::ilo(0), G::ihi(0), t);
+      double xd[G::W];
+#pragma unroll
+      for (int k = 0; k < G::W; k++) xd[k] = u52_to_dbl(x[k]);
+      ring_inv<LOGN, LW, 0>(xd, tw, reinterpret_cast<double *>(lds), W, q, qinv, t);
+#pragma unroll
+      for (int k = 0; k < G::W; k++)
+        out[G::pos(G::iwin(G::R - 1), k, t)] =
+            fp_canon(fp_mulmod(xd[k], ni.x, ni.y, q), qinv, q);
+    } else {
+      const LazyQ Q = lazy_q(M);
+      const u64 *W = rt.psi + ((size_t)p << LOGN), *Ws = rt.psi_sh + ((size_t)p << LOGN);
+      const u64 ni = sn ? sn[si] : rt.ninv[2 * p], nis = sn ? sn[sns + si] : rt.ninv[2 * p + 1];
+      Tw64<LW> tw;
+      ring_tw<LOGN, LW>(tw, W, Ws, G::iwin(0), G::ilo(0), G::ihi(0), t);
+      ring_inv<LOGN, LW, 0>(x, tw, lds, W, Ws, Q, t);
+#pragma unroll
+      for (int k = 0; k < G::W; k++)
+        out[G::pos(G::iwin(G::R - 1), k, t)] = shoup_mul(x[k], ni, nis, Q.q);
+    }
+  }
+}
+
+// Words of target (prime index pt, column tc of the table) converted from ns
+// source limbs of k_ring_ntt's table form (k_basis_convert's words: the
+// centered form's cnt [-Q]_t joins the sum before its reduction, ns 2^60 t +
+// ns t < t 2^64), window at flo(0)
+template <int LOGN, int LW>
+__device__ __forceinline__ void ring_convert(u64 (&x)[1 << LW], const u64 *__restrict__ in,
+                                             int ns, int nd, const u64 *__restrict__ tab,
+                                             int src_prime0, int tc, int pt, bool centered,
+                                             const ModQ *__restrict__ mods, int t) {
+  using G = Ring<LOGN, LW>;
+  u64 hi[G::W], lo[G::W];
+  u32 cnt[G::W];
+#pragma unroll
+  for (int k = 0; k < G::W; k++) hi[k] = lo[k] = cnt[k] = 0;
+  const u64 *hm = tab + 2 * ns;
+  for (int s = 0; s < ns; s++) {
+    const u64 half = (mods[src_prime0 + s].q - 1) / 2, m = hm[s * nd + tc];
+    const u64 *ps = in + ((size_t)s << LOGN);
+#pragma unroll
+    for (int k = 0; k < G::W; k++) {
+      const u64 v = ps[G::pos(G::flo(0), k, t)];
+      cnt[k] += v > half ? 1 : 0;
+      mac_wide(hi[k], lo[k], v, m);
+    }
+  }
+  const ModQ M = mods[pt];
+  const u64 nqm = centered ? to_mont(M.q - hm[(size_t)ns * nd + tc], M) : 0;
+#pragma unroll
+  for (int k = 0; k < G::W; k++) {
+    if (centered) mac_wide(hi[k], lo[k], cnt[k], nqm);
+    x[k] = redc(hi[k], lo[k], M.q, M.qinv);
+  }
+}
+
+// ModUp of every digit: blocks (limb l of E, digit, item).  coeff: per item
+// [limbs][N] coefficients; ext: per item [digits][E][N]; a digit's own limbs
+// are copied from own (own_copy) or skipped.
+template <int LOGN, int LW>
+__global__ __launch_bounds__((1 << (LOGN - LW))) void k_ring_modup(
+    Strided coeff, Strided ext, Batch own, int own_copy, int limbs, int E, int ds, int L,
+    RingDigits dg, RingTabs rt) {
+  using G = Ring<LOGN, LW>;
+  __shared__ u64 lds[G::kLds];
+  const int t = threadIdx.x, l = blockIdx.x, j = blockIdx.y, it = blockIdx.z;
+  const int lo = j * ds, hi = min(lo + ds, limbs), ns = hi - lo;
+  u64 *out = ext.base + it * ext.stride + (((size_t)j * E + l) << LOGN);
+  if (l >= lo && l < hi) {
+    if (own_copy) {
+      const u64 *o = batch_ptr(own, it) + ((size_t)l << LOGN);
+#pragma unroll
+      for (int k = 0; k < G::W; k++) out[t + G::T * k] = o[t + G::T * k];
+    }
+    return;
+  }
+  const int p = prime_of(l, limbs, L);
+  u64 x[G::W];
+  ring_convert<LOGN, LW>(x, coeff.base + it * coeff.stride + ((size_t)lo << LOGN), ns, E - ns,
+                         dg.tab[j], lo, l < lo ? l : l - ns, p, false, rt.mods, t);
+  ring_forward<LOGN, LW>(x, lds, rt, p, t);
+#pragma unroll
+  for (int k = 0; k < G::W; k++) out[t + G::T * k] = x[k];
+}
+
+// ModDown and combine: blocks (limb, component, item).  sp: per (item,
+// component) the alpha special limbs as coefficients; acc: per item
+// [2][E][N]; out = (acc - NTT(conv)) P^-1 + add[sigma(k)] + plus[k].
+struct RingModDown {
+  Strided sp, acc;
+  const u64 *pinv, *tab;
+  int limbs, E, alpha, L;
+  RingItem it[kMaxBatch];
+};
+template <int LOGN, int LW>
+__global__ __launch_bounds__((1 << (LOGN - LW))) void k_ring_moddown(RingModDown a, RingTabs rt) {
+  using G = Ring<LOGN, LW>;
+  __shared__ u64 lds[G::kLds];
+  const int t = threadIdx.x, l = blockIdx.x, comp = blockIdx.y, it = blockIdx.z;
+  const RingItem io = a.it[it];
+  const u64 q = rt.mods[l].q;
+  const u64 *ac = a.acc.base + it * a.acc.stride + (((size_t)comp * a.E + l) << LOGN) + t;
+  const u64 *ad = comp ? io.add1 : io.add0;
+  const u64 *pl = io.plus ? io.plus + (((size_t)comp * a.limbs + l) << LOGN) + t : nullptr;
+  u64 *o = (comp ? io.out1 : io.out0) + ((size_t)l << LOGN) + t;
+  const u64 pinv = a.pinv[2 * l], pinvs = a.pinv[2 * l + 1], g = io.galois;
+  u64 x[G::W], d[G::W], e[G::W];
+  // the combine's operands, loaded ahead of the transform where the
+  // registers hold them
+  auto load = [&] {
+#pragma unroll
+    for (int k = 0; k < G::W; k++) {
+      const u32 j = t + G::T * k;
+      d[k] = ad ? ad[((size_t)l << LOGN) + (g == 1 ? j : autom_index(j, g, LOGN))] : 0;
+      e[k] = ac[G::T * k];
+    }
+  };
+  if constexpr (kEarly<LW>) load();
+  ring_convert<LOGN, LW>(x, a.sp.base + (2 * it + comp) * a.sp.stride, a.alpha, a.limbs, a.tab,
+                         a.L, l, l, true, rt.mods, t);
+  ring_forward<LOGN, LW>(x, lds, rt, l, t);
+  if constexpr (!kEarly<LW>) load();
+#pragma unroll
+  for (int k = 0; k < G::W; k++) d[k] = add_mod(d[k], pl ? pl[G::T * k] : 0, q);
+#pragma unroll
+  for (int k = 0; k < G::W; k++)
+    o[G::T * k] = add_mod(shoup_mul(sub_mod(e[k], x[k], q), pinv, pinvs, q), d[k], q);
+}
+
+static RingTabs ring_tabs(const ckks_context *c, bool inverse) {
+  return RingTabs{c->d_mods, inverse ? c->d_ipsi : c->d_psi, inverse ? c->d_ipsi_sh : c->d_psi_sh,
+                  (const double2 *)(inverse ? c->d_itw_fp : c->d_tw_fp), c->d_ninv,
+                  (const double2 *)c->d_ninv_fp};
+}
+
+// F(std::integral_constant<LOGN>, std::integral_constant<LW>): 8 words a
+// thread up to N = 2^13 (1024 threads), 16 at 2^14
+template <typename F>
+static void ring_shape(int logN, F f) {
+  using std::integral_constant;
+  switch (logN) {
+    case 10: f(integral_constant<int, 10>{}, integral_constant<int, 3>{}); break;
+    case 11: f(integral_constant<int, 11>{}, integral_constant<int, 3>{}); break;
+    case 12: f(integral_constant<int, 12>{}, integral_constant<int, 3>{}); break;
+    case 13: f(integral_constant<int, 13>{}, integral_constant<int, 3>{}); break;
+    case 14: f(integral_constant<int, 14>{}, integral_constant<int, 4>{}); break;
+    default: throw std::invalid_argument("whole-ring kernels: N = 2^10 .. 2^14");
+  }
+}
+
+static void ring_ntt(ckks_context *c, const Batch &src, const Batch &dst, int n_items, int l_begin,
+                     int l_count, int q_limbs, bool inverse, const RingDigits &dg = RingDigits{}) {
+  ring_shape(c->logN, [&](auto ln, auto lw) {
+    constexpr int LN = decltype(ln)::value, LW = decltype(lw)::value;
+    auto kern = inverse ? k_ring_ntt<LN, LW, true> : k_ring_ntt<LN, LW, false>;
+    hipLaunchKernelGGL(kern, dim3(l_count, n_items), dim3(1 << (LN - LW)), 0, c->stream, src, dst,
+                       l_begin, q_limbs, c->L, ring_tabs(c, inverse), dg);
+  });
+  LAUNCH_CHECK();
+}
+
+void launch_ring_sources(ckks_context *c, const Batch &src, const Batch &dst, int n_items,
+                         int l_begin, int l_count, int q_limbs, const BCTable *const *tabs,
+                         int per) {
+  KTimer kt(c, "ntt_inv", 16.0 * c->N * n_items * l_count,
+            0.5 * c->N * c->logN * n_items * l_count);
+  RingDigits dg{};
+  dg.per = per;
+  dg.limbs = l_count;
+  for (int j = 0; j * per < l_count; j++) dg.tab[j] = tabs[j]->sn;
+  ring_ntt(c, src, dst, n_items, l_begin, l_count, q_limbs, true, dg);
+}
+
+bool ring_convert_ok(const ckks_context *c, int ns) {
+  return c->logN >= 10 && c->logN <= 14 && ns <= kRingSources;
+}
+
+void launch_ring_modup(ckks_context *c, const Strided &coeff, const Strided &ext, const Batch &own,
+                       bool own_copy, int n_items, int limbs, int digits, const BCTable *const *tabs) {
+  const int E = limbs + c->alpha;
+  KTimer kt(c, "ring_modup", 8.0 * c->N * n_items * (limbs + (double)digits * E),
+            0.5 * c->N * c->logN * n_items * (double)(digits * E - limbs));
+  RingDigits dg{};
+  for (int j = 0; j < digits; j++) dg.tab[j] = tabs[j]->d;
+  ring_shape(c->logN, [&](auto ln, auto lw) {
+    constexpr int LN = decltype(ln)::value, LW = decltype(lw)::value;
+    hipLaunchKernelGGL((k_ring_modup<LN, LW>), dim3(E, digits, n_items), dim3(1 << (LN - LW)), 0,
+                       c->stream, coeff, ext, own, own_copy ? 1 : 0, limbs, E, c->ds, c->L, dg,
+                       ring_tabs(c, false));
+  });
+  LAUNCH_CHECK();
+}
+
+void launch_ring_moddown(ckks_context *c, const Strided &sp, const Strided &acc,
+                         const RingItem *items, int n_items, int limbs, const u64 *pinv,
+                         const BCTable &tab) {
+  if (n_items > kMaxBatch) throw std::invalid_argument("ring ModDown: too many items");
+  KTimer kt(c, "ring_moddown", 8.0 * c->N * 2.0 * n_items * (c->alpha + 3.0 * limbs),
+            0.5 * c->N * c->logN * 2.0 * n_items * limbs);
+  RingModDown a{sp, acc, pinv, tab.d, limbs, limbs + c->alpha, c->alpha, c->L, {}};
+  std::copy(items, items + n_items, a.it);
+  ring_shape(c->logN, [&](auto ln, auto lw) {
+    constexpr int LN = decltype(ln)::value, LW = decltype(lw)::value;
+    hipLaunchKernelGGL((k_ring_moddown<LN, LW>), dim3(limbs, 2, n_items), dim3(1 << (LN - LW)), 0,
+                       c->stream, a, ring_tabs(c, false));
+  });
+  LAUNCH_CHECK();
+}
+
 template <int S1, int S2, int TILE>
 static void ntt_dispatch(ckks_context *c, const Batch &src, const Batch &dst, int n_items,
                          int l_begin, int l_count, int q_limbs, bool inverse) {
@@ -1201,11 +1747,11 @@ void launch_ntt(ckks_context *c, const Batch &src, const Batch &dst, int n_items
             0.5 * c->N * c->logN * n_items * l_count);
   if (n_items <= 0 || l_count <= 0) return;
   switch (c->logN) {
-    case 10: ntt_dispatch<5, 5, 1024>(c, src, dst, n_items, l_begin, l_count, q_limbs, inverse); break;
-    case 11: ntt_dispatch<5, 6, 2048>(c, src, dst, n_items, l_begin, l_count, q_limbs, inverse); break;
-    case 12: ntt_dispatch<6, 6, 4096>(c, src, dst, n_items, l_begin, l_count, q_limbs, inverse); break;
-    case 13: ntt_dispatch<6, 7, 4096>(c, src, dst, n_items, l_begin, l_count, q_limbs, inverse); break;
-    case 14: ntt_dispatch<7, 7, 4096>(c, src, dst, n_items, l_begin, l_count, q_limbs, inverse); break;
+    case 10:
+    case 11:
+    case 12:
+    case 13:
+    case 14: ring_ntt(c, src, dst, n_items, l_begin, l_count, q_limbs, inverse); break;
     case 15: ntt_dispatch<7, 8, 4096>(c, src, dst, n_items, l_begin, l_count, q_limbs, inverse); break;
     case 16: ntt16_dispatch(c, src, dst, n_items, l_begin, l_count, q_limbs, inverse); break;
     case 17: ntt_dispatch<8, 9, 4096>(c, src, dst, n_items, l_begin, l_count, q_limbs, inverse); break;
@@ -3613,6 +4159,74 @@ void launch_key_inner(ckks_context *c, const Batch &ext, const Batch &acc, int n
   LAUNCH_CHECK();
 }
 
+// k_key_inner of up to 64 jobs of one item each, every job with a key, an
+// automorphism and an extended item of its own (hoisted rotations of one
+// ciphertext), in one launch: grid (N / 256, E, jobs)
+struct InnerJobs {
+  const u64 *key[kMaxBatch];
+  u64 galois[kMaxBatch];
+  int item[kMaxBatch];
+};
+
+template <int MD>
+__global__ __launch_bounds__(TPB) void k_key_inner_jobs(Strided ext, Strided acc, InnerJobs jb,
+                                                        int digits, int E, int q_limbs, int L,
+                                                        int K, int logN,
+                                                        const ModQ *__restrict__ mods, Batch own,
+                                                        int has_own, int ds) {
+  const int k = blockIdx.x * TPB + threadIdx.x;
+  const int l = blockIdx.y, job = blockIdx.z, it = jb.item[job];
+  const int p = prime_of(l, q_limbs, L);
+  const ModQ M = mods[p];
+  const size_t N = (size_t)1 << logN;
+  const u64 g = jb.galois[job];
+  const u32 kk = g == 1 ? (u32)k : autom_index((u32)k, g, logN);
+  const u64 *key = jb.key[job] + (size_t)p * N + key_slot(kk);
+  const u64 *e = ext.base + it * ext.stride + (size_t)l * N + kk;
+  const int jo = (has_own && l < q_limbs) ? l / ds : -1;
+  u64 x[MD], kb[MD], ka[MD];
+#pragma unroll
+  for (int j = 0; j < MD; j++) {
+    if (j < digits) {
+      x[j] = j == jo ? batch_ptr(own, it)[(size_t)l * N + kk] : e[(size_t)j * E * N];
+      kb[j] = key[(size_t)(2 * j) * K * N];
+      ka[j] = key[(size_t)(2 * j + 1) * K * N];
+    }
+  }
+  u64 h0 = 0, l0 = 0, h1 = 0, l1 = 0;
+#pragma unroll
+  for (int j = 0; j < MD; j++) {
+    if (j < digits) {
+      mac_wide(h0, l0, x[j], kb[j]);
+      mac_wide(h1, l1, x[j], ka[j]);
+    }
+  }
+  u64 *a = acc.base + job * acc.stride;
+  a[(size_t)l * N + k] = redc(h0, l0, M.q, M.qinv);
+  a[((size_t)E + l) * N + k] = redc(h1, l1, M.q, M.qinv);
+}
+
+void launch_key_inner_jobs(ckks_context *c, const Strided &ext, const Strided &acc, int n_jobs,
+                           const int *items, const DeviceKey *const *keys, const u64 *galois,
+                           int digits, int E, int q_limbs, const Batch *own) {
+  KTimer kt(c, "key_inner", 8.0 * c->N * n_jobs * (digits * E + 2.0 * E + 2.0 * digits * E),
+            2.0 * c->N * E * digits * n_jobs);
+  if (n_jobs > kMaxBatch) throw std::invalid_argument("key inner product: too many jobs");
+  InnerJobs jb{};
+  for (int i = 0; i < n_jobs; i++) {
+    audit_keyswitch(c, 1, 1, q_limbs, digits, E);
+    jb.key[i] = keys[i]->data;
+    jb.galois[i] = galois[i];
+    jb.item[i] = items[i];
+  }
+  Batch ob{};
+  if (own) ob = *own;
+  auto kern = digits <= 4 ? k_key_inner_jobs<4> : k_key_inner_jobs<kMaxDigits>;
+  hipLaunchKernelGGL(kern, dim3(c->N / TPB, E, n_jobs), dim3(TPB), 0, c->stream, ext, acc, jb,
+                     digits, E, q_limbs, c->L, c->K, c->logN, c->d_mods, ob, own ? 1 : 0, c->ds);
+  LAUNCH_CHECK();
+}
+
 // ===========================================================================
 // Key inner products of several rotations sharing one ModUp (hoisted babies),
 // written before ModDown in the Q u P basis:
@@ -3994,6 +4608,45 @@ void launch_mac(ckks_context *c, const Batch &babies, const Batch &pts, int B, u
   dim3 grid(c->N / TPB, limbs_total, 2);
   hipLaunchKernelGGL(k_mac, grid, dim3(TPB), 0, c->stream, babies, pts, B, out, c->logN,
                      limbs_total, q_limbs, c->L, c->d_mods);
+  LAUNCH_CHECK();
+}
+
+// k_mac of G groups sharing the babies (plaintext of group g and baby b at
+// pts.p[g B + b], outputs [G][2][limbs][N]) in one launch: a small ring's
+// group is a few blocks a limb.  grid (N / 256, limbs, 2 G)
+struct MacGroupPts {
+  const u64 *p[kMacGroupPts];
+};
+
+__global__ void k_mac_groups(Batch babies, MacGroupPts pts, int B, u64 *__restrict__ out, int logN,
+                             int limbs, const ModQ *__restrict__ mods) {
+  const int k = blockIdx.x * TPB + threadIdx.x;
+  const int l = blockIdx.y, comp = blockIdx.z & 1, g = blockIdx.z >> 1;
+  const size_t N = (size_t)1 << logN;
+  const ModQ M = mods[l];
+  const size_t off = ((size_t)comp * limbs + l) * N + k, po = (size_t)l * N + k;
+  u64 acc = 0;
+  for (int b0 = 0; b0 < B; b0 += 16) {
+    const int nb = min(16, B - b0);
+    u64 hi = 0, lo = 0;
+#pragma unroll 8
+    for (int b = 0; b < nb; b++)
+      mac_wide(hi, lo, batch_ptr(babies, b0 + b)[off], pts.p[g * B + b0 + b][po]);
+    acc = add_mod(acc, redc(hi, lo, M.q, M.qinv), M.q);
+  }
+  out[(size_t)g * 2 * limbs * N + off] = to_mont(acc, M);
+}
+
+void launch_mac_groups(ckks_context *c, const Batch &babies, const u64 *const *pts, int B, int G,
+                       u64 *out, int limbs) {
+  KTimer kt(c, "mac", 8.0 * c->N * limbs * (B * (G + 2.0) + 2.0 * G),
+            2.0 * c->N * limbs * B * G);
+  if (B * G > kMacGroupPts) throw std::invalid_argument("MAC groups: too many plaintexts");
+  audit_pt(c, (double)B * G * limbs);
+  MacGroupPts mp{};
+  for (int i = 0; i < B * G; i++) mp.p[i] = pts[i];
+  hipLaunchKernelGGL(k_mac_groups, dim3(c->N / TPB, limbs, 2 * G), dim3(TPB), 0, c->stream, babies,
+                     mp, B, out, c->logN, limbs, c->d_mods);
   LAUNCH_CHECK();
 }
 

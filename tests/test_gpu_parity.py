@@ -361,6 +361,43 @@ def test_bsgs_matvec_parity():
     assert np.abs(dec - W @ x).max() < 1e-5
 
 
+@pytest.mark.parametrize("params,B,G", [
+    # digits of 4 primes (converted inside the whole-ring kernels), and more
+    # giant groups than one pass holds
+    (dict(log_n=10, depth=7, dnum=2, dcrt_bits=40, first_mod=60, special_bits=60), 3, 67),
+    # digits of 5 (converted before the transforms), wide primes only
+    (dict(log_n=11, depth=4, dnum=1, dcrt_bits=59, first_mod=60, special_bits=60), 2, 3),
+    # more plaintexts than one launch of the MACs takes; 3-prime digits, the last of 1
+    (dict(log_n=12, depth=3, dnum=2, dcrt_bits=59, first_mod=60, special_bits=60), 40, 8),
+    # the largest whole-ring transform, both arithmetic paths
+    (dict(log_n=14, depth=4, dnum=3, dcrt_bits=40, first_mod=40, special_bits=60), 2, 2),
+])
+def test_small_ring_keyswitch_shapes_parity(params, B, G):
+    """Hoisted babies, group MACs and giant key switches of rings below 2^15
+    at every level: limbs equal to the oracle's."""
+    fhe = _fhe()
+    rots = list(range(1, B)) + [B]
+    client, ctx, orc = _pair(params, rotations=tuple(rots))
+    rng = np.random.default_rng(params["log_n"])
+    slots = 32
+    for limbs in sorted({ctx.L, ctx.L - 1, 1}, reverse=True):
+        sc = ctx.scale_at(limbs)
+        z = rng.uniform(-1, 1, slots)
+        ct = client.encrypt(z, slots=slots, cur_limbs=limbs, enc_id=7)
+        ref = orc.encrypt(z, slots=slots, scale=sc, limbs=limbs, enc_id=7)
+        rows = rng.uniform(-1, 1, (B * G, slots))
+        pts = fhe.encode_rows(ctx, rows, limbs=limbs, scale=sc, slots=slots)
+        rpts = np.stack([orc.encode(r, slots=slots, scale=sc, limbs=limbs) for r in rows])
+        babies = fhe.prepare_hoisted_baby_rotations(ct, list(range(B)), ctx)
+        rb = orc.hoisted_rotate(ref, [orc.galois_elt(b) for b in range(B)])
+        for b in range(B):
+            assert np.array_equal(babies[b].download(), rb[b]), (limbs, b)
+        acc = fhe.hoisted_mac_sum(ct, list(range(B)), pts, B, G, ctx)
+        racc = orc.hoisted_mac_sum(ref, [orc.galois_elt(b) for b in range(B)], rpts,
+                                   orc.galois_elt(B), G)
+        assert np.array_equal(acc.download(), racc), limbs
+
+
 @pytest.mark.parametrize("name", ["matvec", "ext44"])
 def test_bsgs_matvec_ext_parity(name):
     """The matvec workload with strategy "ext_normal": babies in Q u P, one
