@@ -1056,6 +1056,10 @@ static bool ks_modup(ckks_context *c, int limbs, int n, const u64 *const *d, u64
     const size_t est = (size_t)digits * E * N;
     const bool packed = pack && high_only && !own_copy;
     launch_ntt_inv_low(c, src, strided(coeff, (size_t)limbs * N), n, 0, limbs, limbs, dmul);
+    const BCTable *tabs[kMaxDigits];
+    for (int j = 0; j < digits; j++) tabs[j] = &bc_up(c, limbs, j);
+    launch_convert_h4_digits(c, strided(coeff, (size_t)limbs * N), strided(ext, est), n, tabs,
+                             digits, limbs, packed);
     for (int j = 0; j < digits; j++) {
       const int lo = j * c->ds, hi = std::min((j + 1) * c->ds, limbs), ns = hi - lo;
       u64 *ej = ext + (size_t)j * E * N;
@@ -1064,8 +1068,6 @@ static bool ks_modup(ckks_context *c, int limbs, int n, const u64 *const *d, u64
         for (int i = 0; i < n; i++) dsrc.p[i] = (u64 *)d[i] + (size_t)lo * N;
         launch_copy_limbs(c, dsrc, strided(ej + (size_t)lo * N, est), n, ns);
       }
-      launch_convert_h4(c, strided(coeff + (size_t)lo * N, (size_t)limbs * N), strided(ej, est),
-                        n, bc_up(c, limbs, j), lo, lo, ns, limbs, false, packed);
       if (!high_only) {
         launch_ntt_fwd_low(c, strided(ej, est), n, 0, lo, limbs);
         launch_ntt_fwd_low(c, strided(ej, est), n, hi, E - hi, limbs);
@@ -1102,6 +1104,10 @@ static bool ks_modup(ckks_context *c, int limbs, int n, const u64 *const *d, u64
   return false;
 }
 
+// A batched key switch is split into parts of at least this many items
+// (run_parts)
+constexpr int kSplitMin = 8;
+
 struct KsJob {
   int ext_item;
   const DeviceKey *key;
@@ -1118,6 +1124,7 @@ struct KsDeferred {
   // where ks_moddown's tile conversion applies)
   int below = -1;
   bool on = false;
+  int from = 0;  // the limbs deferred: fp64 ones from here on
   const u64 *ext = nullptr;
   size_t est = 0;
   Batch own{};
@@ -1201,10 +1208,10 @@ static void ks_moddown(ckks_context *c, int limbs, u64 *acc, const std::vector<K
       launch_low_key_moddown(c, dk->ext, dk->est, dk->own, n, *dk->key, dk->digits, E, limbs,
                              dk->ginv, strided(conv, (size_t)limbs * N), pinv,
                              pmod_table(c, limbs), a0, add1_off, o0, out1_off, limbs,
-                             nullptr, dk->own_b, dk->packed);
+                             nullptr, dk->own_b, dk->packed, dk->from);
     launch_ntt_moddown(c, strided(conv, (size_t)limbs * N), n, limbs, strided(acc, 2 * E * N), E,
                        pinv, a0, add1_off, gal.data(), o0, out1_off, nullptr, nullptr, tile,
-                       deferred);
+                       deferred ? dk->from : limbs);
     return;
   }
   if (deferred) throw std::logic_error("deferred key product without the fused combine");
@@ -1278,6 +1285,27 @@ static u64 galois_inverse(const ckks_context *c, u64 g) {
   return inv;
 }
 
+// The fp64 Q limbs from the returned one on go through the fused key product +
+// combine (16 n blocks a limb, two blocks a CU), the others through the
+// special limbs' launch and the separate combine (which q_0 takes anyway).
+// All of them, unless a last round of few blocks can move whole into the free
+// slots of the special limbs' launch: one ciphertext of 35 fp64 limbs is 560
+// blocks, 48 more than run at once, and 84 us against 65 us with 3 limbs
+// moved (the other two launches 3 us longer).
+static int defer_from(const ckks_context *c, int n, int limbs) {
+  if (n >= 2 * kSplitMin) return 0;  // parts on other streams fill the gaps
+  const int slots = 2 * kCUs, per = 16 * n;
+  int fp = 0, other = c->alpha;
+  for (int l = 0; l < limbs; l++) (c->prime_fp[l] ? fp : other)++;
+  const int rest = fp * per % slots;
+  if (fp * per < slots || rest == 0) return 0;
+  const int move = (rest + per - 1) / per, room = (slots - other * per % slots) % slots;
+  if (move * per > room || move >= fp) return 0;
+  int from = 0;
+  for (int left = move; left > 0; from++) left -= c->prime_fp[from];
+  return from;
+}
+
 // ModUp of n polynomials d[i] (NTT domain) and the key inner product of
 // every job (job i takes ext item i; all share one key and Galois element)
 // into [n][2][E][N] accumulators.  At N = 2^16 the extended digits get only
@@ -1315,6 +1343,7 @@ static u64 *ks_modup_inner(ckks_context *c, int limbs, int n, const u64 *const *
   if (dk) {
     dk->on = defer;
     if (defer) {
+      dk->from = dk->below >= 0 ? 0 : defer_from(c, n, limbs);
       dk->ext = ext;
       dk->est = est;
       dk->own = ob;
@@ -1327,7 +1356,7 @@ static u64 *ks_modup_inner(ckks_context *c, int limbs, int n, const u64 *const *
   }
   launch_ntt_low_key(c, ext, est, ob, acc, 2 * (size_t)E * N, n, *jobs[0].key, digits, E, limbs,
                      ginv, spf ? sp : nullptr, defer ? (dk->below >= 0 ? dk->below : limbs) : 0,
-                     dmul, packed);
+                     dmul, packed, defer ? dk->from : 0);
   return acc;
 }
 
@@ -1378,8 +1407,6 @@ static void gen_key(ckks_context *c, u64 id, int relin, u64 galois) {
 // back before the function returns; every part's intermediates stay
 // allocated until then, so that no block of one part is handed to another
 // while still in use.  Parts keep at least kSplitMin items.
-constexpr int kSplitMin = 8;
-
 struct StreamSwap {
   ckks_context *c;
   hipStream_t saved;
@@ -1613,7 +1640,8 @@ static void relin_rescale_batch(ckks_context *c, const ckks_ct *const *in, int n
                                ta ? fa : d3, P, o0, (u64)T * N, T, ta ? &fb : nullptr,
                                dk.own_b, dk.packed);
       launch_ntt_moddown(c, strided(conv, (size_t)T * N), nb, T, strided(acc, 2 * E * N), E, rt,
-                         d3, P, gal.data(), o0, (u64)T * N, amul, &po, tile, dk.on);
+                         d3, P, gal.data(), o0, (u64)T * N, amul, &po, tile,
+                         dk.on ? 0 : T);
     } else {
       Batch a1{}, o1{};
       for (int i = 0; i < nb; i++) {

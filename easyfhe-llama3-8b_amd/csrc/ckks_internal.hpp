@@ -23,6 +23,7 @@ typedef uint32_t u32;
 
 namespace ckks {
 
+constexpr int kCUs = 256;        // compute units of the chip
 constexpr int kMaxBatch = 64;    // explicit pointers per kernel argument block
 constexpr int kMaxDigitSize = 16;  // Montgomery fold bound: 16 * 2^60 <= 2^64
 constexpr int kMaxDigits = 8;
@@ -528,7 +529,7 @@ void launch_ntt_fwd_high(ckks_context *c, const Batch &src, const Batch &dst, in
 // sp.stride + (l - q_limbs) N, and are not written to acc: the ModDown then
 // runs launch_ntt_inv_high on them.
 bool low_key_special_fp(const ckks_context *c);
-// The Q limbs of fp64 primes below defer_below are skipped
+// The Q limbs of fp64 primes of [defer_from, defer_below) are skipped
 // (launch_low_key_moddown runs their key product with the ModDown's combine)
 // With own_b, the digits' own limbs are those of own x own_b (word by word),
 // formed where they are read.
@@ -536,16 +537,16 @@ void launch_ntt_low_key(ckks_context *c, const u64 *ext, size_t ext_stride, cons
                         u64 *acc, size_t acc_stride, int n_items, const DeviceKey &key,
                         int digits, int E, int q_limbs, u64 ginv, const Strided *sp = nullptr,
                         int defer_below = 0, const Batch *own_b = nullptr,
-                        bool ext_packed = false);
+                        bool ext_packed = false, int defer_from = 0);
 // N = 2^16: for the Q limbs of fp64 primes, launch_ntt_low_key's key product
 // and launch_ntt_moddown's combine (addends and outputs as there, no postop)
 // in one kernel, the accumulator kept in the block, for output limbs
-// [0, out_limbs) (q_limbs, or the kept limbs of a relinearise-rescale, whose
+// [from, out_limbs) (q_limbs, or the kept limbs of a relinearise-rescale, whose
 // pinv is (P p_1..p_D)^-1); conv holds the ModDown's conversion after the
 // forward high pass (launch_convert_h4), 2 n items of out_limbs limbs; pmod
 // per Q limb [P]_q and its Shoup constant.  The special limbs' key product
 // and the other Q limbs run through launch_ntt_low_key(defer_below) and
-// launch_ntt_moddown(wide_only).
+// launch_ntt_moddown(deferred_from).
 // With mul_b, add and mul_b are the factors a and b of the degree-2
 // products whose d0 = a0 b0 and d1 = a0 b1 + a1 b0 (a1, b1 at add1_off)
 // are the addend, formed in the kernel (launch_tensor then writes the d0 /
@@ -555,7 +556,7 @@ void launch_low_key_moddown(ckks_context *c, const u64 *ext, size_t ext_stride, 
                             u64 ginv, const Batch &conv, const u64 *pinv, const u64 *pmod,
                             const Batch &add, u64 add1_off, const Batch &out, u64 out1_off,
                             int out_limbs, const Batch *mul_b = nullptr,
-                            const Batch *own_b = nullptr, bool ext_packed = false);
+                            const Batch *own_b = nullptr, bool ext_packed = false, int from = 0);
 // N = 2^16: the high pass of the inverse NTT alone, in place (after the low
 // pass of launch_ntt_low_key's sp output)
 void launch_ntt_inv_high(ckks_context *c, const Batch &dst, int n_items, int l_begin, int l_count,
@@ -566,12 +567,13 @@ void launch_moddown_combine(ckks_context *c, const Strided &acc, const Strided &
                             int E, const u64 *pinv, const u64 *amul = nullptr,
                             const PostOp *post = nullptr);
 // high_done: conv already went through the forward high pass
-// (launch_convert_h4), only the low pass with the combine runs
+// (launch_convert_h4), only the low pass with the combine runs; fp64 limbs
+// from deferred_from on are left to launch_low_key_moddown
 void launch_ntt_moddown(ckks_context *c, const Batch &conv, int n, int limbs, const Batch &acc,
                         int E, const u64 *pinv, const Batch &add, u64 add1_off,
                         const u64 *galois, const Batch &out, u64 out1_off,
                         const u64 *amul = nullptr, const PostOp *post = nullptr,
-                        bool high_done = false, bool wide_only = false);
+                        bool high_done = false, int deferred_from = 1 << 30);
 // the forward NTT's low pass alone, in place (N = 2^16: after the high pass of
 // launch_convert_h4 or launch_ntt_fwd_high)
 void launch_ntt_fwd_low(ckks_context *c, const Batch &data, int n_items, int l_begin,
@@ -600,6 +602,10 @@ void launch_convert_h4_rs(ckks_context *c, const Batch &src, const Batch &dst, i
 void launch_convert_h4(ckks_context *c, const Batch &src, const Batch &dst, int n_items,
                        const BCTable &t, int src_prime0, int t_split, int t_skip, int q_limbs,
                        bool centered, bool packed = false);
+// launch_convert_h4 of every digit of a ModUp: src per item [q_limbs][N], dst
+// per item [digits][E][N], tabs the digits' tables
+void launch_convert_h4_digits(ckks_context *c, const Batch &src, const Batch &dst, int n_items,
+                              const BCTable *const *tabs, int digits, int q_limbs, bool packed);
 void launch_rescale_lift(ckks_context *c, const Batch &last, const Batch &w, int n_items,
                          int limbs, int D, const u64 *tab);
 void launch_rescale_finish(ckks_context *c, const Batch &src, const Batch &w, const Batch &out,

@@ -4,6 +4,8 @@
 // uint64 limb arrays of N residues; the NTT domain is the bit-reversed
 // evaluation order a_hat[i] = a(psi^(2 br(i) + 1)).
 #include <math.h>
+
+#include <algorithm>
 #include <type_traits>
 
 #include "ckks_internal.hpp"
@@ -1773,13 +1775,11 @@ void launch_ntt_inv_high(ckks_context *c, const Batch &dst, int n_items, int l_b
 void launch_ntt_moddown(ckks_context *c, const Batch &conv, int n, int limbs, const Batch &acc,
                         int E, const u64 *pinv, const Batch &add, u64 add1_off,
                         const u64 *galois, const Batch &out, u64 out1_off, const u64 *amul,
-                        const PostOp *post, bool high_done, bool wide_only) {
-  // the limbs this call combines (wide_only: those of primes at or above 2^45)
-  int run_limbs = limbs;
-  if (wide_only) {
-    run_limbs = 0;
-    for (int l = 0; l < limbs; l++) run_limbs += c->prime_fp[l] ? 0 : 1;
-  }
+                        const PostOp *post, bool high_done, int deferred_from) {
+  // the limbs this call combines
+  auto runs = [&](int l) { return l < deferred_from || !c->prime_fp[l]; };
+  int run_limbs = 0;
+  for (int l = 0; l < limbs; l++) run_limbs += runs(l) ? 1 : 0;
   KTimer kt(c, "ntt_fwd_moddown",
             8.0 * c->N * run_limbs *
                 (6.0 * n + (batch_ptr_host(add, 0) ? (add1_off ? 2.0 : 1.0) * n : 0.0)),
@@ -1797,15 +1797,14 @@ void launch_ntt_moddown(ckks_context *c, const Batch &conv, int n, int limbs, co
   if (post) md.post = *post;
   for (int i = 0; i < n; i++) md.gal.g[i] = galois[i];
   if (!high_done) launch_fwd_high16(c, conv, conv, 2 * n, 0, limbs, limbs);
-  // runs of limbs (wide_only: the limbs of primes at or above 2^45 alone,
-  // the others being combined by launch_low_key_moddown)
+  // runs of limbs (the others are combined by launch_low_key_moddown)
   for (int l0 = 0; l0 < limbs;) {
-    if (wide_only && c->prime_fp[l0]) {
+    if (!runs(l0)) {
       l0++;
       continue;
     }
     int l1 = l0 + 1;
-    while (l1 < limbs && !(wide_only && c->prime_fp[l1])) l1++;
+    while (l1 < limbs && runs(l1)) l1++;
     hipLaunchKernelGGL(k_ntt16m_fwd_low<true>, dim3(16, 2 * n, l1 - l0), dim3(TPB), 0, c->stream,
                        conv, l0, limbs, c->L, c->d_mods, c->d_psi, c->d_psi_sh,
                        (const double2 *)c->d_tw_fp, md);
@@ -2194,6 +2193,33 @@ __global__ __launch_bounds__(TPB, 2) void k_ntt16_low_key(LowKeyArgs a, int l_be
     low_key_64(lds, a, it, tile, l, p, mods, psi, psi_sh);
 }
 
+// The same over runs of limbs of several kinds in one launch (the bodies'
+// register allocations all stay at two waves per SIMD, so the runs share the
+// chip instead of following one another: one ciphertext, 12 special limbs and
+// q_0: 38 + 28 us in two launches, 38 us in one)
+struct LowKeyRuns {
+  int begin[3], count[3], kind[3];  // kind: 0 64-bit, 1 fp64, 2 fp64 with SPINV
+  int n;
+};
+
+__global__ __launch_bounds__(TPB, 2) void k_ntt16_low_key_runs(
+    LowKeyArgs a, LowKeyRuns runs, int n_items, const ModQ *__restrict__ mods,
+    const u64 *__restrict__ psi, const u64 *__restrict__ psi_sh, const double2 *__restrict__ tw,
+    const double2 *__restrict__ rinv) {
+  __shared__ u64 lds[16 * 272];
+  const int b = blockIdx.x, r = b >> 3;
+  const int it = r % n_items, tl = (r / n_items) * 8 + (b & 7);
+  const int tile = tl & 15;
+  int i = tl >> 4, k = 0;
+  while (k + 1 < runs.n && i >= runs.count[k]) i -= runs.count[k++];
+  const int l = runs.begin[k] + i, kind = runs.kind[k];
+  const int p = prime_of(l, a.q_limbs, a.L);
+  if (kind == 0) low_key_64(lds, a, it, tile, l, p, mods, psi, psi_sh);
+  else if (kind == 1)
+    low_key_fp<false>(reinterpret_cast<double *>(lds), a, it, tile, l, p, mods, tw, rinv);
+  else low_key_fp<true>(reinterpret_cast<double *>(lds), a, it, tile, l, p, mods, tw, rinv);
+}
+
 // ===========================================================================
 // N = 2^16, fp64 Q limbs: the key product of one (item, tile, limb) and the
 // ModDown's combine of the output tile it maps to, with the accumulator kept
@@ -2416,7 +2442,7 @@ void launch_low_key_moddown(ckks_context *c, const u64 *ext, size_t ext_stride, 
                             u64 ginv, const Batch &conv, const u64 *pinv, const u64 *pmod,
                             const Batch &add, u64 add1_off, const Batch &out, u64 out1_off,
                             int out_limbs, const Batch *mul_b, const Batch *own_b,
-                            bool ext_packed) {
+                            bool ext_packed, int from) {
   if (n_items <= 0) return;
   if (n_items > kMaxBatch) throw std::invalid_argument("fused key product + ModDown: n <= 64");
   if (out_limbs < 1 || out_limbs > q_limbs)
@@ -2444,7 +2470,7 @@ void launch_low_key_moddown(ckks_context *c, const u64 *ext, size_t ext_stride, 
             2.0 * c->N * out_limbs * digits * n_items +
                 0.5 * c->N * 12 * 2.0 * n_items * out_limbs +
                 (md.prod ? 3.0 * c->N * n_items * out_limbs : 0.0));
-  for (int l0 = 0; l0 < out_limbs;) {
+  for (int l0 = from; l0 < out_limbs;) {
     if (!c->prime_fp[l0]) {
       l0++;
       continue;
@@ -2462,7 +2488,8 @@ void launch_low_key_moddown(ckks_context *c, const u64 *ext, size_t ext_stride, 
 void launch_ntt_low_key(ckks_context *c, const u64 *ext, size_t ext_stride, const Batch &own,
                         u64 *acc, size_t acc_stride, int n_items, const DeviceKey &key,
                         int digits, int E, int q_limbs, u64 ginv, const Strided *sp,
-                        int defer_below, const Batch *own_b, bool ext_packed) {
+                        int defer_below, const Batch *own_b, bool ext_packed,
+                        int defer_from) {
   KTimer kt(c, "ntt_low_key",
             8.0 * c->N * ((double)n_items * (digits * E + 2.0 * E) + 2.0 * digits * E),
             2.0 * c->N * E * digits * n_items);
@@ -2480,26 +2507,48 @@ void launch_ntt_low_key(ckks_context *c, const u64 *ext, size_t ext_stride, cons
   // primes the 64-bit one)
   // (with sp, the special limbs (all fp64) form a run of their own)
   auto fp_limb = [&](int l) { return c->prime_fp[l < q_limbs ? l : c->L + (l - q_limbs)] != 0; };
-  // (kind 3: fp64 Q limbs below defer_below, left to launch_low_key_moddown)
+  // (kind 3: fp64 Q limbs of [defer_from, defer_below), left to
+  // launch_low_key_moddown)
   auto kind = [&](int l) {
-    return fp_limb(l) ? (sp && l >= q_limbs ? 2 : (l < defer_below ? 3 : 1)) : 0;
+    return fp_limb(l) ? (sp && l >= q_limbs ? 2 : (l >= defer_from && l < defer_below ? 3 : 1)) : 0;
   };
+  struct Run {
+    int begin, count, kind;
+  };
+  std::vector<Run> all;
   for (int l0 = 0; l0 < E;) {
     const int k = kind(l0);
     int l1 = l0 + 1;
     while (l1 < E && kind(l1) == k) l1++;
-    if (k == 3) {
-      l0 = l1;
-      continue;
+    if (k != 3) all.push_back(Run{l0, l1 - l0, k});
+    l0 = l1;
+  }
+  if (all.size() == 2 || all.size() == 3) {
+    // the 64-bit run first: its blocks take the longest
+    std::stable_sort(all.begin(), all.end(), [](const Run &x, const Run &y) { return !x.kind && y.kind; });
+    LowKeyRuns runs{};
+    int limbs = 0;
+    for (const Run &r : all) {
+      runs.begin[runs.n] = r.begin;
+      runs.count[runs.n] = r.count;
+      runs.kind[runs.n++] = r.kind;
+      limbs += r.count;
     }
+    hipLaunchKernelGGL(k_ntt16_low_key_runs, dim3(n_items * 16 * limbs), dim3(TPB), 0, c->stream, a,
+                       runs, n_items, c->d_mods, c->d_psi, c->d_psi_sh,
+                       (const double2 *)c->d_tw_fp, (const double2 *)c->d_rinv_fp);
+    LAUNCH_CHECK();
+    return;
+  }
+  for (const Run &r : all) {
+    const int k = r.kind;
     auto kern = k == 2 ? k_ntt16_low_key<true, true>
                 : k == 1 ? k_ntt16_low_key<true, false>
                          : k_ntt16_low_key<false, false>;
-    hipLaunchKernelGGL(kern, dim3(n_items * 16 * (l1 - l0)), dim3(TPB), 0, c->stream, a, l0, n_items,
-                       c->d_mods, c->d_psi, c->d_psi_sh, (const double2 *)c->d_tw_fp,
+    hipLaunchKernelGGL(kern, dim3(n_items * 16 * r.count), dim3(TPB), 0, c->stream, a, r.begin,
+                       n_items, c->d_mods, c->d_psi, c->d_psi_sh, (const double2 *)c->d_tw_fp,
                        (const double2 *)c->d_rinv_fp);
     LAUNCH_CHECK();
-    l0 = l1;
   }
 }
 
@@ -3245,12 +3294,35 @@ struct H4Tabs {
 // and row; each kept target t < nd - RSD then adds
 // r_j [P p_1..p_j]_t - (r_j > p_(j+1) / 2 ? [P p_1..p_(j+1)]_t : 0) before
 // its forward high pass.  rs / rsf: launch_bc_down_rescale's tables.
+//
+// One launch takes several conversions of the same number of source quads
+// (every digit of a ModUp): blockIdx.z = job split + part.  A part is a range
+// of the job's passes, so that few items still fill the chip: a block's time
+// is one wave's chain of source columns and passes, and 64 blocks a job and
+// item leave most CUs idle.  Parts repeat the source columns (about one
+// pass's work), so the launcher splits only below two blocks a CU.  One
+// ciphertext, three digits of 12 primes into 36: 165 us in three launches, now
+// 51 us; its ModDown, 2 x 12 into 36: 55 -> 36 us.
+struct H4Job {
+  const u64 *tab, *mtab;  // BCTable::sn, mt
+  u64 src_off, dst_off;   // words from an item of src / dst
+  int ns, nd, n_tg, wide_mask, src_prime0, t_split, t_skip, flags;
+};
+struct H4Jobs {
+  H4Job j[kMaxDigits];
+};
 template <int NK, int RSD = 0>
 __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
-    Batch src, Batch dst, int ns, int nd, const u64 *__restrict__ tab,
-    const u64 *__restrict__ mtab, int n_tg, int wide_mask, int src_prime0, int t_split,
-    int t_skip, int q_limbs, int L, int flags, const ModQ *__restrict__ mods, H4Tabs nt,
-    const u64 *__restrict__ rs, const double2 *__restrict__ rsf) {
+    Batch src, Batch dst, H4Jobs jobs, int split, int q_limbs, int L,
+    const ModQ *__restrict__ mods, H4Tabs nt, const u64 *__restrict__ rs,
+    const double2 *__restrict__ rsf) {
+  const int part = blockIdx.z % split;
+  const H4Job &jb = jobs.j[blockIdx.z / split];
+  const u64 *__restrict__ tab = jb.tab;
+  const u64 *__restrict__ mtab = jb.mtab;
+  const int ns = jb.ns, nd = jb.nd, n_tg = jb.n_tg, wide_mask = jb.wide_mask;
+  const int src_prime0 = jb.src_prime0, t_split = jb.t_split, t_skip = jb.t_skip;
+  const int flags = jb.flags;
   constexpr bool RS = RSD > 0;
   constexpr int TW = bc_tgt_words(RSD);
   const int T = nd - RSD;
@@ -3263,14 +3335,32 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
   extern __shared__ u64 tb[];
   const int lane = threadIdx.x & 63, g = lane >> 4, col = lane & 15, wave = threadIdx.x >> 6;
   const int cc = blockIdx.x * 64 + wave * 16 + col;
-  const u64 *in = batch_ptr(src, blockIdx.y) + cc;
-  u64 *out = batch_ptr(dst, blockIdx.y) + cc;
+  const u64 *in = batch_ptr(src, blockIdx.y) + jb.src_off + cc;
+  u64 *out = batch_ptr(dst, blockIdx.y) + jb.dst_off + cc;
+  // this part's passes [p0, p1) of 8 targets each; RS: the last pass holds
+  // the dropped targets, runs first in every part, and part 0 stores its kept
+  // targets
+  const int n_pass = (nd + 7) >> 3, n_div = RS ? n_pass - 1 : n_pass;
+  const int p0 = n_div * part / split, p1 = n_div * (part + 1) / split;
+  auto mine = [&](int t) {
+    const int p = t >> 3;
+    return (p >= p0 && p < p1) || (RS && p == n_pass - 1);
+  };
   // the table and per-target constants (k_basis_convert_mfma's words, and
   // the target's prime index at word 9)
   const int words = NK * n_tg * 512;
-  for (int idx = threadIdx.x; idx < words; idx += TPB) tb[idx] = mtab[idx];
+  if (split == 1) {
+    for (int idx = threadIdx.x; idx < words; idx += TPB) tb[idx] = mtab[idx];
+  } else {
+    for (int b = 0; b < NK * n_tg; b++) {
+      const int t0 = 16 * (b % n_tg);
+      if (!mine(t0) && !mine(t0 + 8)) continue;
+      for (int idx = threadIdx.x; idx < 512; idx += TPB) tb[b * 512 + idx] = mtab[b * 512 + idx];
+    }
+  }
   u64 *tgt = tb + words;
   for (int t = threadIdx.x; t < nd; t += TPB) {
+    if (!mine(t) && t) continue;  // target 0 stands in for lanes past nd
     const int tl = t < t_split ? t : t + t_skip;
     const int pt = prime_of(tl, q_limbs, L);
     const ModQ M = mods[pt];
@@ -3310,6 +3400,7 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
   for (int idx = threadIdx.x; idx < (nd + ns) * 16; idx += TPB) {
     const int t = idx >> 4, j = idx & 15;
     const bool src_side = t >= nd;
+    if (!src_side && !mine(t)) continue;
     int pt;
     if (src_side) {
       pt = src_prime0 + (t - nd);
@@ -3396,11 +3487,10 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
   // MFMA output (targets 16 tg + 4 e + g), so that a lane keeps two target
   // columns (y) beside its sources (a) in registers; each pass recomputes
   // the group's MFMAs.  RS: the pass of the dropped targets goes first.
-  const int first = RS ? ((nd - 1) >> 3) : 0;  // = 2 tg + h of the last target
-  for (int pp = 0; pp < 2 * n_tg; pp++) {
-    const int pq = RS ? (pp == 0 ? first : (pp <= first ? pp - 1 : pp)) : pp;
+  for (int pp = RS ? p0 - 1 : p0; pp < p1; pp++) {
+    const bool lifts = RS && pp == p0 - 1;
+    const int pq = lifts ? n_pass - 1 : pp;
     const int tg = pq >> 1, h = pq & 1;
-    if (16 * tg + 8 * h >= nd) continue;  // no target in this pass
     const bool wide = (wide_mask >> tg) & 1;
     // lane m + 16 k supplies row m of the table operand; reading row
     // (m & 12) | ((m + 2 h) & 3) instead puts targets 16 tg + 4 (2 h + ee) + g
@@ -3472,7 +3562,7 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
       }
     }
     if constexpr (RS) {
-      if (pp == 0) {
+      if (lifts) {
         // the lifts, in the lanes of each dropped target (fp64 primes; the
         // transposed order puts target t in lane group t % 4, row t % 16 / 4)
         const u64 *rpinv = rs + 2 * (size_t)T * RSD;
@@ -3513,6 +3603,7 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
           }
           __syncthreads();
         }
+        if (part) continue;
       }
       // every kept target adds its lifts
 #pragma unroll
@@ -3600,9 +3691,13 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
 // high pass of such targets after it (target t at output limb
 // t < t_split ? t : t + t_skip).  Each returns the kernel's flag (2, 4) when
 // the launch is mixed, else 0 and runs nothing: a launch of wide primes only
-// keeps its high passes inside.
+// keeps its high passes inside.  So does one of few items (one ciphertext's
+// digits, or its two ModDown components): there a launch of 16 blocks an item
+// costs 5 us and the waiting lanes 1 to 2.
+constexpr int kH4Inside = 2;
 static int h4_wide_sources(ckks_context *c, const Batch &src, int n_items, int ns,
                            int src_prime0, int q_limbs) {
+  if (n_items <= kH4Inside) return 0;
   int wide = 0;
   for (int s = 0; s < ns; s++) wide += c->prime_fp[src_prime0 + s] ? 0 : 1;
   if (wide == 0 || wide == ns) return 0;
@@ -3635,6 +3730,7 @@ static int h4_wide_targets(ckks_context *c, const Batch &dst, int n_items, int n
     return !c->prime_fp[tl < q_limbs ? tl : c->L + (tl - q_limbs)];
   };
   int n_wide = 0;
+  if (n_items <= kH4Inside) return 0;
   for (int t = 0; t < n_out; t++) n_wide += wide(t) ? 1 : 0;
   if (n_wide == 0 || n_wide == n_out) return 0;
   if (!run) return 4;
@@ -3661,6 +3757,39 @@ bool convert_h4_ok(const ckks_context *c, const BCTable &t) {
          t.n_tg <= 4 && t.nd <= 64 && convert_h4_lds(t) <= 65536;
 }
 
+// parts of a launch's passes: as many as run at once (two blocks a CU); more
+// parts start a second round that costs what it saves (one ciphertext's three
+// digits, 192 blocks: 2 parts 51 us, 3 parts 55 us)
+static int h4_split(int blocks, int passes) {
+  return std::max(1, std::min(2 * kCUs / blocks, passes));
+}
+
+static H4Tabs h4_tabs(const ckks_context *c) {
+  return H4Tabs{c->d_psi, c->d_psi_sh, c->d_ipsi, c->d_ipsi_sh, c->d_ninv,
+                (const double2 *)c->d_tw_fp, (const double2 *)c->d_itw_fp,
+                (const double2 *)c->d_ninv_fp};
+}
+
+static Batch batch_at(const Batch &b, int n_items, u64 off) {
+  Batch r = b;
+  if (r.base) r.base += off;
+  else
+    for (int i = 0; i < n_items; i++) r.p[i] += off;
+  return r;
+}
+
+static void h4_launch(ckks_context *c, const Batch &src, const Batch &dst, int n_items,
+                      const H4Jobs &jobs, int n_jobs, int n_k, size_t lds, int q_limbs) {
+  int passes = 0;
+  for (int j = 0; j < n_jobs; j++) passes = std::max(passes, (jobs.j[j].nd + 7) >> 3);
+  const int split = h4_split(64 * n_items * n_jobs, passes);
+  auto kern = n_k == 1 ? k_convert_h4<1, 0> : n_k == 2 ? k_convert_h4<2, 0> : k_convert_h4<3, 0>;
+  hipLaunchKernelGGL(kern, dim3(64, n_items, n_jobs * split), dim3(TPB), lds, c->stream, src, dst,
+                     jobs, split, q_limbs, c->L, c->d_mods, h4_tabs(c), (const u64 *)nullptr,
+                     (const double2 *)nullptr);
+  LAUNCH_CHECK();
+}
+
 void launch_convert_h4(ckks_context *c, const Batch &src, const Batch &dst, int n_items,
                        const BCTable &t, int src_prime0, int t_split, int t_skip, int q_limbs,
                        bool centered, bool packed) {
@@ -3668,19 +3797,73 @@ void launch_convert_h4(ckks_context *c, const Batch &src, const Batch &dst, int 
             (double)c->N * n_items * t.ns * t.nd);
   if (!convert_h4_ok(c, t)) throw std::invalid_argument("tile-resident conversion: shape");
   if (n_items <= 0) return;
-  auto kern = t.n_k == 1 ? k_convert_h4<1, 0> : t.n_k == 2 ? k_convert_h4<2, 0> : k_convert_h4<3, 0>;
-  const size_t lds = convert_h4_lds(t);
-  H4Tabs nt{c->d_psi, c->d_psi_sh, c->d_ipsi, c->d_ipsi_sh, c->d_ninv,
-            (const double2 *)c->d_tw_fp, (const double2 *)c->d_itw_fp,
-            (const double2 *)c->d_ninv_fp};
   const int flags = (centered ? 1 : 0) | (packed ? 8 : 0) |
                     h4_wide_sources(c, src, n_items, t.ns, src_prime0, q_limbs) |
                     h4_wide_targets(c, dst, n_items, t.nd, t_split, t_skip, q_limbs, false);
-  hipLaunchKernelGGL(kern, dim3(64, n_items), dim3(TPB), lds, c->stream, src, dst, t.ns, t.nd,
-                     t.sn, t.mt, t.n_tg, t.wide_mask, src_prime0, t_split, t_skip, q_limbs, c->L,
-                     flags, c->d_mods, nt, (const u64 *)nullptr, (const double2 *)nullptr);
-  LAUNCH_CHECK();
+  H4Jobs jobs{};
+  jobs.j[0] = H4Job{t.sn, t.mt, 0, 0, t.ns, t.nd, t.n_tg, t.wide_mask, src_prime0, t_split, t_skip,
+                    flags};
+  h4_launch(c, src, dst, n_items, jobs, 1, t.n_k, convert_h4_lds(t), q_limbs);
   if (flags & 4) h4_wide_targets(c, dst, n_items, t.nd, t_split, t_skip, q_limbs, true);
+}
+
+void launch_convert_h4_digits(ckks_context *c, const Batch &src, const Batch &dst, int n_items,
+                              const BCTable *const *tabs, int digits, int q_limbs, bool packed) {
+  if (n_items <= 0) return;
+  const int E = q_limbs + c->alpha;
+  double bytes = 0.0, ops = 0.0;
+  for (int j = 0; j < digits; j++) {
+    if (!convert_h4_ok(c, *tabs[j])) throw std::invalid_argument("tile-resident conversion: shape");
+    bytes += 8.0 * c->N * n_items * (tabs[j]->ns + tabs[j]->nd);
+    ops += (double)c->N * n_items * tabs[j]->ns * tabs[j]->nd;
+  }
+  KTimer kt(c, "convert_h4", bytes, ops);
+  H4Jobs all{};
+  // digits by the limb ranges of their wide targets' high passes
+  std::map<std::pair<int, int>, std::vector<int>> wide;
+  auto is_wide = [&](int l) { return !c->prime_fp[l < q_limbs ? l : c->L + (l - q_limbs)]; };
+  for (int j = 0; j < digits; j++) {
+    const BCTable &t = *tabs[j];
+    const int lo = j * c->ds;
+    const u64 so = (u64)lo << 16, po = ((u64)j * E) << 16;
+    const Batch sj = batch_at(src, n_items, so), dj = batch_at(dst, n_items, po);
+    const int flags = (packed ? 8 : 0) | h4_wide_sources(c, sj, n_items, t.ns, lo, q_limbs) |
+                      h4_wide_targets(c, dj, n_items, t.nd, lo, t.ns, q_limbs, false);
+    all.j[j] = H4Job{t.sn, t.mt, so, po, t.ns, t.nd, t.n_tg, t.wide_mask, lo, lo, t.ns, flags};
+    if (!(flags & 4)) continue;
+    auto own = [&](int l) { return l >= lo && l < lo + t.ns; };
+    for (int l = 0; l < E; l++) {
+      if (own(l) || !is_wide(l)) continue;
+      int l1 = l + 1;
+      while (l1 < E && !own(l1) && is_wide(l1)) l1++;
+      wide[{l, l1}].push_back(j);
+      l = l1 - 1;
+    }
+  }
+  for (int j = 0; j < digits;) {
+    // a run of digits with one count of source quads
+    int j1 = j + 1;
+    while (j1 < digits && tabs[j1]->n_k == tabs[j]->n_k) j1++;
+    H4Jobs jobs{};
+    size_t lds = 0;
+    for (int i = j; i < j1; i++) {
+      jobs.j[i - j] = all.j[i];
+      lds = std::max(lds, convert_h4_lds(*tabs[i]));
+    }
+    h4_launch(c, src, dst, n_items, jobs, j1 - j, tabs[j]->n_k, lds, q_limbs);
+    j = j1;
+  }
+  for (const auto &w : wide) {
+    std::vector<u64 *> items;
+    for (int i = 0; i < n_items; i++)
+      for (int j : w.second) items.push_back(batch_ptr_host(dst, i) + (((size_t)j * E) << 16));
+    for (size_t i0 = 0; i0 < items.size(); i0 += kMaxBatch) {
+      const int nb = (int)std::min(items.size() - i0, (size_t)kMaxBatch);
+      Batch b{};
+      for (int i = 0; i < nb; i++) b.p[i] = items[i0 + i];
+      launch_fwd_high16(c, b, b, nb, w.first.first, w.first.second - w.first.first, q_limbs);
+    }
+  }
 }
 
 bool convert_h4_rs_ok(const ckks_context *c, const BCTable &t, int D) {
@@ -3704,14 +3887,13 @@ void launch_convert_h4_rs(ckks_context *c, const Batch &src, const Batch &dst, i
       (const double2 *)(rtab + 2 * (size_t)T * D + 2 * (size_t)D + 3 * (size_t)D * D);
   auto k1 = t.n_k == 1 ? k_convert_h4<1, 1> : t.n_k == 2 ? k_convert_h4<2, 1> : k_convert_h4<3, 1>;
   auto k2 = t.n_k == 1 ? k_convert_h4<1, 2> : t.n_k == 2 ? k_convert_h4<2, 2> : k_convert_h4<3, 2>;
-  H4Tabs nt{c->d_psi, c->d_psi_sh, c->d_ipsi, c->d_ipsi_sh, c->d_ninv,
-            (const double2 *)c->d_tw_fp, (const double2 *)c->d_itw_fp,
-            (const double2 *)c->d_ninv_fp};
   const int flags = 1 | h4_wide_sources(c, src, n_items, t.ns, c->L, t.nd) |
                     h4_wide_targets(c, dst, n_items, T, t.nd, 0, t.nd, false);
-  hipLaunchKernelGGL(D == 1 ? k1 : k2, dim3(64, n_items), dim3(TPB), convert_h4_lds(t, D),
-                     c->stream, src, dst, t.ns, t.nd, t.sn, t.mt, t.n_tg, t.wide_mask, c->L,
-                     t.nd, 0, t.nd, c->L, flags, c->d_mods, nt, rtab, rsf);
+  H4Jobs jobs{};
+  jobs.j[0] = H4Job{t.sn, t.mt, 0, 0, t.ns, t.nd, t.n_tg, t.wide_mask, c->L, t.nd, 0, flags};
+  const int passes = (t.nd + 7) >> 3, split = h4_split(64 * n_items, std::max(1, passes - 1));
+  hipLaunchKernelGGL(D == 1 ? k1 : k2, dim3(64, n_items, split), dim3(TPB), convert_h4_lds(t, D),
+                     c->stream, src, dst, jobs, split, t.nd, c->L, c->d_mods, h4_tabs(c), rtab, rsf);
   LAUNCH_CHECK();
   if (flags & 4) h4_wide_targets(c, dst, n_items, T, t.nd, 0, t.nd, true);
 }

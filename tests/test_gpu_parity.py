@@ -768,6 +768,42 @@ def test_keyswitch_kernel_choices_full_size(env, monkeypatch):
     ctx.close()
 
 
+@pytest.mark.slow
+@pytest.mark.parametrize("params,levels", [
+    # fp64 limbs and q_0: levels with and without limbs moved out of the fused
+    # combine, whole and split conversions, one to three digits
+    ("keyswitch", (36, 34, 25, 12, 3)),
+    # wide primes only, digits of 5 and 2 primes (two source-quad counts)
+    (dict(log_n=16, depth=9, dnum=2, dcrt_bits=59, first_mod=60, special_bits=60), (10, 7, 2)),
+    # fp64 limbs between wide q_0 and wide special primes
+    (dict(log_n=16, depth=9, dnum=2, dcrt_bits=40, first_mod=60, special_bits=60), (10, 6)),
+])
+def test_keyswitch_small_batches_full_size(params, levels):
+    """Rotations and products of 1, 2, 3 and 5 ciphertexts at N = 2^16: the
+    conversions' parts and the moved limbs depend on the batch; the words are
+    the oracle's at every size."""
+    fhe = _fhe()
+    r = 1 << 7
+    client, ctx, orc = _pair(params, rotations=(r,))
+    slots = 64
+    rng = np.random.default_rng(12)
+    zs = [rng.uniform(-1, 1, slots) for _ in range(5)]
+    for limbs in levels:
+        cts = [client.encrypt(z, slots=slots, cur_limbs=limbs, enc_id=400 + i)
+               for i, z in enumerate(zs)]
+        refs = [orc.encrypt(z, slots=slots, scale=ctx.scale_at(limbs), limbs=limbs, enc_id=400 + i)
+                for i, z in enumerate(zs)]
+        rot = [orc.rotate_g(x, orc.galois_elt(r)) for x in refs]
+        prod = [orc.rescale(orc.relinearize(orc.tensor(refs[i], refs[i - 1]))) for i in range(5)]
+        for n in (1, 2, 3, 5):
+            for got, want in zip(fhe.homo_rotate_many(cts[:n], r, ctx), rot):
+                assert np.array_equal(got.download(), want), (limbs, n)
+            got = fhe.homo_mul_relin_rescale_many(cts[:n], [cts[i - 1] for i in range(n)], ctx)
+            for i in range(n):
+                assert np.array_equal(got[i].download(), prod[i]), (limbs, n, i)
+    ctx.close()
+
+
 def test_linear_combination_matches_composed_ops():
     """One fused launch = mul_scalar + add + add_scalar on the same words,
     with terms holding more limbs than the output."""
