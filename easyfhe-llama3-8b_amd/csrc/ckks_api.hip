@@ -1114,7 +1114,7 @@ struct KsJob {
   u64 galois;
   const u64 *add0, *add1;
   u64 *out0, *out1;
-  const u64 *plus = nullptr;  // [2][limbs][N] added as it is (ring_convert_ok(alpha) only)
+  const u64 *plus = nullptr;  // [2][limbs][N] added as it is (all jobs of a ModDown or none)
 };
 
 // The key product of the fp64 Q limbs left by ks_modup_inner for ks_moddown
@@ -1173,8 +1173,22 @@ static void ks_moddown(ckks_context *c, int limbs, u64 *acc, const std::vector<K
     }
     return;
   }
+  // the added ciphertexts, through the combines' postop or the fused combine
+  const bool has_plus = jobs[0].plus != nullptr;
   for (const KsJob &jb : jobs)
-    if (jb.plus) throw std::logic_error("ModDown: added ciphertexts on the ring path only");
+    if ((jb.plus != nullptr) != has_plus) throw std::logic_error("ModDown: mixed added ciphertexts");
+  auto plus_of = [&](int b0, int nb) {
+    Batch b{};
+    for (int i = 0; i < nb; i++) b.p[i] = (u64 *)jobs[b0 + i].plus;
+    return b;
+  };
+  auto post_of = [&](int b0, int nb) {
+    PostOp po{};
+    po.sub = plus_of(b0, nb);
+    po.sub1_off = (u64)limbs * N;
+    po.plus = 1;
+    return po;
+  };
   u64 *conv = s.get((size_t)n * 2 * limbs * N);
   // N = 2^16: the special limbs' inverse high pass, the conversion and the
   // forward high pass of the Q limbs in one kernel, then the low pass with
@@ -1204,13 +1218,19 @@ static void ks_moddown(ckks_context *c, int limbs, u64 *acc, const std::vector<K
       o0.p[i] = jobs[i].out0;
       gal[i] = jobs[i].galois;
     }
+    // the fused combine adds at the outputs' component offset
+    if (has_plus && out1_off != (u64)limbs * N) throw std::logic_error("ModDown: added layout");
+    const Batch pl = plus_of(0, n);
+    const PostOp po = post_of(0, n);
     if (deferred)
       launch_low_key_moddown(c, dk->ext, dk->est, dk->own, n, *dk->key, dk->digits, E, limbs,
                              dk->ginv, strided(conv, (size_t)limbs * N), pinv,
                              pmod_table(c, limbs), a0, add1_off, o0, out1_off, limbs,
-                             nullptr, dk->own_b, dk->packed, dk->from);
+                             nullptr, dk->own_b, dk->packed, dk->from,
+                             has_plus ? &pl : nullptr);
     launch_ntt_moddown(c, strided(conv, (size_t)limbs * N), n, limbs, strided(acc, 2 * E * N), E,
-                       pinv, a0, add1_off, gal.data(), o0, out1_off, nullptr, nullptr, tile,
+                       pinv, a0, add1_off, gal.data(), o0, out1_off, nullptr,
+                       has_plus ? &po : nullptr, tile,
                        deferred ? dk->from : limbs);
     return;
   }
@@ -1231,7 +1251,9 @@ static void ks_moddown(ckks_context *c, int limbs, u64 *acc, const std::vector<K
     }
     Strided sacc{acc + (size_t)b0 * 2 * E * N, 2 * E * N};
     Strided sconv{conv + (size_t)b0 * 2 * limbs * N, 2 * limbs * N};
-    launch_moddown_combine(c, sacc, sconv, a0, a1, gal.data(), o0, o1, nb, limbs, E, pinv);
+    const PostOp po = post_of(b0, nb);
+    launch_moddown_combine(c, sacc, sconv, a0, a1, gal.data(), o0, o1, nb, limbs, E, pinv, nullptr,
+                           has_plus ? &po : nullptr);
   }
 }
 
@@ -1454,9 +1476,12 @@ static size_t rotate_scratch_words(const ckks_context *c, int limbs, int nb) {
 // Rotations of n ciphertexts at one level by the same Galois element.  With
 // `arena` given, every intermediate lives in that fixed buffer of
 // `arena_words` words (n <= 64) and nothing is allocated.
+// With `plus`, ciphertext i of [2][limbs][N] words at plus + i plus_stride is
+// added to rotation i.
 static void rotate_batch(ckks_context *c, const ckks_ct *const *in, int n, u64 g, ckks_ct **out,
                          u64 *arena = nullptr, size_t arena_words = 0,
-                         size_t *arena_used = nullptr) {
+                         size_t *arena_used = nullptr, const u64 *plus = nullptr,
+                         size_t plus_stride = 0) {
   const int limbs = in[0]->limbs;
   const size_t N = c->N, P = (size_t)limbs * N;
   const DeviceKey &key = get_key(c, g);
@@ -1465,7 +1490,8 @@ static void rotate_batch(ckks_context *c, const ckks_ct *const *in, int n, u64 g
     for (int i = 0; i < nb; i++) d[i] = in[b0 + i]->d + P;
     std::vector<KsJob> jobs(nb);
     for (int i = 0; i < nb; i++)
-      jobs[i] = KsJob{i, &key, g, in[b0 + i]->d, nullptr, out[b0 + i]->d, out[b0 + i]->d + P};
+      jobs[i] = KsJob{i, &key, g, in[b0 + i]->d, nullptr, out[b0 + i]->d, out[b0 + i]->d + P,
+                      plus ? plus + (size_t)(b0 + i) * plus_stride : nullptr};
     u64 *ptmp = s.get((size_t)nb * 2 * c->alpha * N);
     const Strided sp{ptmp, (u64)c->alpha * N};
     bool sp_done = false;
@@ -2694,6 +2720,45 @@ int ckks_hoisted_rotate_many(ckks_context *c, const ckks_ct *const *a, int m,
   API_END
 }
 
+// out[i] = a[i] + b[i] for n degree-1 ciphertexts at `limbs` limbs, 64 pairs
+// per launch (the giant Horner chains' adds)
+// (item i's second operand at b + i b_stride)
+static void add_batched(ckks_context *c, const std::vector<ckks_ct *> &a, const u64 *b,
+                        size_t b_stride, ckks_ct *const *out, int n, int limbs) {
+  for (int b0 = 0; b0 < n; b0 += kMaxBatch) {
+    const int nb = std::min(kMaxBatch, n - b0);
+    Batch ba{}, bb{}, bo{};
+    for (int i = 0; i < nb; i++) {
+      ba.p[i] = a[b0 + i]->d;
+      bb.p[i] = (u64 *)(b + (size_t)(b0 + i) * b_stride);
+      bo.p[i] = out[b0 + i]->d;
+    }
+    launch_addsub_many(c, ba, bb, bo, nb, 2, limbs, limbs, 0);
+  }
+}
+
+// One step of a giant Horner chain: cts[i] = rot(cts[i]) + (the ciphertext at
+// add + i stride), the rotations batched and the sum taken in their ModDown
+// (a launch of its own read and wrote each ciphertext once more: 120 us for 16
+// of 13 limbs, 4% of a 4096 x 4096 product)
+static void horner_step(ckks_context *c, ckks_ct **cts, int n, u64 gg, const u64 *add,
+                        size_t stride) {
+  const int limbs = cts[0]->limbs;
+  if (gg == 1) {
+    add_batched(c, std::vector<ckks_ct *>(cts, cts + n), add, stride, cts, n, limbs);
+    return;
+  }
+  std::vector<const ckks_ct *> cur(cts, cts + n);
+  std::vector<ckks_ct *> next(n);
+  for (int i = 0; i < n; i++)
+    next[i] = new_ct(c, 2, limbs, 0, cts[i]->slots, cts[i]->scale, cts[i]->scale_degree);
+  rotate_batch(c, cur.data(), n, gg, next.data(), nullptr, 0, nullptr, add, stride);
+  for (int i = 0; i < n; i++) {
+    free_ct(cts[i]);
+    cts[i] = next[i];
+  }
+}
+
 int ckks_hoisted_mac_sum(ckks_context *c, const ckks_ct *const *babies, int B,
                          const ckks_ct *const *pts, int64_t giant_rotation, int giant_count,
                          ckks_ct **out) {
@@ -2766,35 +2831,10 @@ int ckks_hoisted_mac_sum(ckks_context *c, const ckks_ct *const *babies, int B,
       continue;
     }
     launch_mac(c, bb, bp, B, inner, limbs, limbs);
-    ckks_ct *rot = new_ct(c, 2, limbs, 0, acc->slots, scale, sdeg);
-    if (gg == 1)
-      HIPCHECK(hipMemcpyAsync(rot->d, acc->d, acc->bytes, hipMemcpyDeviceToDevice, c->stream));
-    else {
-      const ckks_ct *ac = acc;
-      rotate_batch(c, &ac, 1, gg, &rot);
-    }
-    launch_addsub(c, rot->d, inner, acc->d, 2, limbs, limbs, 0);
-    free_ct(rot);
+    horner_step(c, &acc, 1, gg, inner, 2 * P);
   }
   *out = acc;
   API_END
-}
-
-// out[i] = a[i] + b[i] for n degree-1 ciphertexts at `limbs` limbs, 64 pairs
-// per launch (the giant Horner chains' adds)
-// (item i's second operand at b + i b_stride)
-static void add_batched(ckks_context *c, const std::vector<ckks_ct *> &a, const u64 *b,
-                        size_t b_stride, ckks_ct *const *out, int n, int limbs) {
-  for (int b0 = 0; b0 < n; b0 += kMaxBatch) {
-    const int nb = std::min(kMaxBatch, n - b0);
-    Batch ba{}, bb{}, bo{};
-    for (int i = 0; i < nb; i++) {
-      ba.p[i] = a[b0 + i]->d;
-      bb.p[i] = (u64 *)(b + (size_t)(b0 + i) * b_stride);
-      bo.p[i] = out[b0 + i]->d;
-    }
-    launch_addsub_many(c, ba, bb, bo, nb, 2, limbs, limbs, 0);
-  }
 }
 
 int ckks_hoisted_mac_sum_many(ckks_context *c, const ckks_ct *const *babies, int n, int B,
@@ -2849,20 +2889,7 @@ int ckks_hoisted_mac_sum_many(ckks_context *c, const ckks_ct *const *babies, int
       }
       continue;
     }
-    // Horner: out = rot(out) + inner_g, the rotations batched over the n
-    std::vector<ckks_ct *> rot(n);
-    for (int i = 0; i < n; i++)
-      rot[i] = new_ct(c, 2, limbs, 0, out[i]->slots, scale, sdeg);
-    if (gg == 1) {
-      for (int i = 0; i < n; i++)
-        HIPCHECK(hipMemcpyAsync(rot[i]->d, out[i]->d, out[i]->bytes, hipMemcpyDeviceToDevice,
-                                c->stream));
-    } else {
-      std::vector<const ckks_ct *> cur(out, out + n);
-      rotate_batch(c, cur.data(), n, gg, rot.data());
-    }
-    add_batched(c, rot, ig, CP, out, n, limbs);
-    for (int i = 0; i < n; i++) free_ct(rot[i]);
+    horner_step(c, out, n, gg, ig, CP);
   }
   API_END
 }
@@ -2871,9 +2898,11 @@ int ckks_hoisted_mac_sum_many(ckks_context *c, const ckks_ct *const *babies, int
 // [2][E][N] before its ModDown: (P c0, P c1) for offset 0,
 // (P sigma(c0) + acc_0, acc_1) otherwise.  One ModUp per ciphertext (batched)
 // is shared by all rotations; each rotation's key is read once for all n.
-// dst[b * n + i] is baby b of ciphertext i.
+// dst[b * n + i] is baby b of ciphertext i.  With id_mask given, the babies
+// of offset 0 are not written but marked there (launch_mac_many reads the
+// ciphertexts).
 static void ext_babies(ckks_context *c, const ckks_ct *const *a, int n, const int64_t *rotations,
-                       int nr, u64 *const *dst, Scratch &s) {
+                       int nr, u64 *const *dst, Scratch &s, u64 *id_mask = nullptr) {
   const int limbs = a[0]->limbs, E = limbs + c->alpha, digits = (limbs + c->ds - 1) / c->ds;
   const size_t N = c->N, P = (size_t)limbs * N, est = (size_t)digits * E * N;
   std::vector<u64> gal(nr);
@@ -2898,7 +2927,9 @@ static void ext_babies(ckks_context *c, const ckks_ct *const *a, int n, const in
   const u64 two_n = 2 * (u64)c->N;
   for (int b = 0; b < nr; b++) {
     if (gal[b] == 1) {
-      for (int i = 0; i < n; i++) launch_ext_identity(c, a[i]->d, dst[b * n + i], limbs);
+      if (id_mask) *id_mask |= (u64)1 << b;
+      else
+        for (int i = 0; i < n; i++) launch_ext_identity(c, a[i]->d, dst[b * n + i], limbs);
       continue;
     }
     rb.push_back(b);
@@ -2911,8 +2942,8 @@ static void ext_babies(ckks_context *c, const ckks_ct *const *a, int n, const in
   }
   if (rb.empty()) return;
   // every rotation of a chunk of ciphertexts in one pass over the digits
-  for (int i0 = 0; i0 < n; i0 += kMultiItems) {
-    const int ni = std::min(kMultiItems, n - i0);
+  for (int i0 = 0; i0 < n; i0 += multi_items(digits)) {
+    const int ni = std::min(multi_items(digits), n - i0);
     std::vector<const u64 *> table(rb.size() * ni);
     for (size_t r = 0; r < rb.size(); r++)
       for (int it = 0; it < ni; it++) table[r * ni + it] = dst[(size_t)rb[r] * n + i0 + it];
@@ -2950,7 +2981,10 @@ static void mac_sum_ext(ckks_context *c, const ckks_ct *const *a, int n,
   u64 *bab = s.get((size_t)B * n * EP);
   std::vector<u64 *> bp((size_t)B * n);
   for (size_t k = 0; k < bp.size(); k++) bp[k] = bab + k * EP;
-  ext_babies(c, a, n, baby_rotations, B, bp.data(), s);
+  u64 id_mask = 0;
+  ext_babies(c, a, n, baby_rotations, B, bp.data(), s, &id_mask);
+  Batch cts{};
+  for (int i = 0; i < n; i++) cts.p[i] = a[i]->d;
   // the MAC of several giant groups runs as one pass over the babies
   const int GC = std::max(1, std::min(kMacGroups, kMaxBatch / B));
   u64 *inner_all = s.get((size_t)std::min(GC, giant_count) * n * EP);
@@ -2964,7 +2998,7 @@ static void mac_sum_ext(ckks_context *c, const ckks_ct *const *a, int n,
       Batch ptb{};
       for (int gi = 0; gi < gn; gi++)
         for (int b = 0; b < B; b++) ptb.p[gi * B + b] = pts[(g_lo + gi) * B + b]->d;
-      launch_mac_many(c, bab, n, ptb, B, gn, inner_all, E, limbs);
+      launch_mac_many(c, bab, n, ptb, B, gn, inner_all, E, limbs, cts, id_mask);
     }
     u64 *inner_ext = inner_all + (size_t)(g - g_lo) * n * EP;
     const bool first = out[0] == nullptr;
@@ -2981,19 +3015,7 @@ static void mac_sum_ext(ckks_context *c, const ckks_ct *const *a, int n,
       ks_moddown(c, limbs, inner_ext, jobs, s2);
     }
     if (first) continue;
-    std::vector<ckks_ct *> rot(n);
-    for (int i = 0; i < n; i++)
-      rot[i] = new_ct(c, 2, limbs, 0, out[i]->slots, out[i]->scale, out[i]->scale_degree);
-    if (gg == 1) {
-      for (int i = 0; i < n; i++)
-        HIPCHECK(hipMemcpyAsync(rot[i]->d, out[i]->d, out[i]->bytes, hipMemcpyDeviceToDevice,
-                                c->stream));
-    } else {
-      std::vector<const ckks_ct *> cur(out, out + n);
-      rotate_batch(c, cur.data(), n, gg, rot.data());
-    }
-    add_batched(c, rot, inner, 2 * P, out, n, limbs);
-    for (int i = 0; i < n; i++) free_ct(rot[i]);
+    horner_step(c, out, n, gg, inner, 2 * P);
   }
 }
 
@@ -3073,7 +3095,10 @@ static void mac_sum_double(ckks_context *c, const ckks_ct *const *a, int n,
   u64 *bab = s.get((size_t)B * n * EP);
   std::vector<u64 *> bp((size_t)B * n);
   for (size_t k = 0; k < bp.size(); k++) bp[k] = bab + k * EP;
-  ext_babies(c, a, n, baby_rotations, B, bp.data(), s);
+  u64 id_mask = 0;
+  ext_babies(c, a, n, baby_rotations, B, bp.data(), s, &id_mask);
+  Batch cts{};
+  for (int i = 0; i < n; i++) cts.p[i] = a[i]->d;
   // inner sums, GC groups per MAC launch, [slot][n][2][E][N]: slot 0 holds
   // group 0's, the running sum; the other groups of a launch go to slots
   // 1..gn (the first launch's to 1..gn-1) and are folded into the sum before
@@ -3089,7 +3114,7 @@ static void mac_sum_double(ckks_context *c, const ckks_ct *const *a, int n,
     Batch ptb{};
     for (int gi = 0; gi < gn; gi++)
       for (int b = 0; b < B; b++) ptb.p[gi * B + b] = pts[(g0 + gi) * B + b]->d;
-    launch_mac_many(c, bab, n, ptb, B, gn, dst, E, limbs);
+    launch_mac_many(c, bab, n, ptb, B, gn, dst, E, limbs, cts, id_mask);
     for (int gi = g0 == 0 ? 1 : 0; gi < gn; gi++) {
       const int g = g0 + gi;
       u64 *ug = dst + (size_t)gi * n * EP;

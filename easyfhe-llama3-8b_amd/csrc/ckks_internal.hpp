@@ -39,7 +39,9 @@ constexpr int kMacGroupPts = 256;   // plaintexts of one launch_mac_groups
 // forms its own sums, about 20 instructions a source and word, against 100 a
 // word for the transform; beyond 4 the separate conversion shares more
 constexpr int kRingSources = 4;
-constexpr int kMultiItems = 4;    // items per multi-rotation key inner product launch
+// items per multi-rotation key inner product launch: 8 ciphertexts share a
+// key word's read where a thread's registers hold their digits
+constexpr int multi_items(int digits) { return digits <= 4 ? 8 : 4; }
 
 // Per-prime constants, resident in device memory.
 struct ModQ {
@@ -69,7 +71,7 @@ struct Strided {
 
 // Epilogue of a relinearise-rescale ModDown (the fused Chebyshev step of
 // homo_mul_relin_rescale_postop): the result r becomes
-//   (dbl ? 2 r : r) - sub + scal   (scal on component 0 only)
+//   (dbl ? 2 r : r) - sub + scal   (scal on component 0 only; + sub with plus)
 // with sub per item at component 0 (null: none), its component 1 at
 // sub + sub1_off, and scal one word per output limb (null: none).
 struct PostOp {
@@ -77,6 +79,7 @@ struct PostOp {
   Batch sub;
   u64 sub1_off;
   const u64 *scal;
+  int plus;
 };
 
 // (both forms are read before the choice, so that a block waits for its
@@ -556,7 +559,8 @@ void launch_low_key_moddown(ckks_context *c, const u64 *ext, size_t ext_stride, 
                             u64 ginv, const Batch &conv, const u64 *pinv, const u64 *pmod,
                             const Batch &add, u64 add1_off, const Batch &out, u64 out1_off,
                             int out_limbs, const Batch *mul_b = nullptr,
-                            const Batch *own_b = nullptr, bool ext_packed = false, int from = 0);
+                            const Batch *own_b = nullptr, bool ext_packed = false, int from = 0,
+                            const Batch *plus = nullptr);
 // N = 2^16: the high pass of the inverse NTT alone, in place (after the low
 // pass of launch_ntt_low_key's sp output)
 void launch_ntt_inv_high(ckks_context *c, const Batch &dst, int n_items, int l_begin, int l_count,
@@ -644,7 +648,7 @@ void launch_mac_table(ckks_context *c, const u64 *const *bab, int n, const u64 *
 // so `src` may be freed on return).
 void upload_async(ckks_context *c, void *dst, const void *src, size_t bytes);
 void launch_mac_many(ckks_context *c, const u64 *bab, int n, const Batch &pts, int B, int G,
-                     u64 *out, int E, int q_limbs);
+                     u64 *out, int E, int q_limbs, const Batch &cts, u64 id_mask);
 void launch_ext_identity(ckks_context *c, const u64 *ct, u64 *out, int limbs);
 void launch_ext_add_pc0(ckks_context *c, const u64 *ct, u64 *out, int limbs, u64 galois);
 void launch_moddown_one(ckks_context *c, const Batch &src, Strided conv, const Batch &out,

@@ -409,7 +409,10 @@ __device__ __forceinline__ u64 apply_post(const PostOp &po, int item, int comp, 
                                           size_t N, u64 r, u64 q) {
   if (po.dbl) r = add_mod(r, r, q);
   const u64 *sb = batch_ptr(po.sub, item);
-  if (sb) r = sub_mod(r, sb[(comp ? po.sub1_off : 0) + (size_t)limb * N + e], q);
+  if (sb) {
+    const u64 s = sb[(comp ? po.sub1_off : 0) + (size_t)limb * N + e];
+    r = po.plus ? add_mod(r, s, q) : sub_mod(r, s, q);
+  }
   if (po.scal && !comp) r = add_mod(r, po.scal[limb], q);
   return r;
 }
@@ -472,7 +475,7 @@ __device__ __forceinline__ void md_store(const MDCombine &md, int item2, int lim
   if (md.amul) d = shoup_mul(d, pf.am, pf.ams, q);
   r = add_mod(r, d, q);
   if (md.post.dbl) r = add_mod(r, r, q);
-  r = sub_mod(r, s, q);
+  r = md.post.plus ? add_mod(r, s, q) : sub_mod(r, s, q);
   if (pf.sc) r = add_mod(r, pf.sc, q);
   u64 *o = batch_ptr(md.out, item) + (comp ? md.out1_off : 0);
   o[(size_t)limb * N + e] = r;
@@ -2248,9 +2251,12 @@ struct LowMD {
   Batch out;
   u64 out1_off;
   int prod;
+  Batch plus;  // per item [2 x out1_off] words added to the outputs (null: none)
 };
 
-
+// PLUS: md.plus is added; an instance of its own, so that the plain one
+// keeps its register allocation.
+template <bool PLUS>
 __global__ __launch_bounds__(TPB, 2) void k_low_key_md(LowKeyArgs a, LowMD md, Batch conv,
                                                        const u64 *__restrict__ pmod,
                                                        int l_begin, int n_items,
@@ -2391,13 +2397,25 @@ __global__ __launch_bounds__(TPB, 2) void k_low_key_md(LowKeyArgs a, LowMD md, B
     row_sync();
 #pragma unroll
     for (int j = 0; j < 16; j++) sm[lds16(rl, 16 * c0 + j)] = x[j];
-    row_sync();
-    u64 *o = batch_ptr(md.out, it) + (comp ? md.out1_off : 0) + ((size_t)l << 16);
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
+    const size_t oo = (comp ? md.out1_off : 0) + ((size_t)l << 16) + e0;
+    u64 *o = batch_ptr(md.out, it) + oo;
+    auto value = [&](int k) {
       const double acc = comp ? acc1t[lds16(rl, c0 + 16 * k)] : av[k];
-      const double v = __dsub_rn(acc, sm[lds16(rl, c0 + 16 * k)]);
-      o[e0 + 16 * k] = fp_canon(fp_mulmod(v, pinv, pinvq, q), qinv, q);
+      return fp_mulmod(__dsub_rn(acc, sm[lds16(rl, c0 + 16 * k)]), pinv, pinvq, q);
+    };
+    if constexpr (PLUS) {
+      const u64 *pl = batch_ptr(md.plus, it) + oo;
+      u64 pw[16];
+#pragma unroll
+      for (int k = 0; k < 16; k++) pw[k] = pl[16 * k];
+      row_sync();
+#pragma unroll
+      for (int k = 0; k < 16; k++)  // in [-q, 2q] with the added word
+        o[16 * k] = fp_canon(__dadd_rn(value(k), u52_to_dbl(pw[k])), qinv, q);
+    } else {
+      row_sync();
+#pragma unroll
+      for (int k = 0; k < 16; k++) o[16 * k] = fp_canon(value(k), qinv, q);
     }
   }
 }
@@ -2442,7 +2460,7 @@ void launch_low_key_moddown(ckks_context *c, const u64 *ext, size_t ext_stride, 
                             u64 ginv, const Batch &conv, const u64 *pinv, const u64 *pmod,
                             const Batch &add, u64 add1_off, const Batch &out, u64 out1_off,
                             int out_limbs, const Batch *mul_b, const Batch *own_b,
-                            bool ext_packed, int from) {
+                            bool ext_packed, int from, const Batch *plus) {
   if (n_items <= 0) return;
   if (n_items > kMaxBatch) throw std::invalid_argument("fused key product + ModDown: n <= 64");
   if (out_limbs < 1 || out_limbs > q_limbs)
@@ -2455,6 +2473,7 @@ void launch_low_key_moddown(ckks_context *c, const u64 *ext, size_t ext_stride, 
   md.add1_off = add1_off;
   md.out = out;
   md.out1_off = out1_off;
+  if (plus) md.plus = *plus;
   if (mul_b) {
     if (!batch_ptr_host(add, 0) || !add1_off)
       throw std::invalid_argument("fused key product + ModDown: product addend needs both factors");
@@ -2477,7 +2496,8 @@ void launch_low_key_moddown(ckks_context *c, const u64 *ext, size_t ext_stride, 
     }
     int l1 = l0 + 1;
     while (l1 < out_limbs && c->prime_fp[l1]) l1++;
-    hipLaunchKernelGGL(k_low_key_md, dim3(n_items * 16 * (l1 - l0)), dim3(TPB), 0, c->stream, a,
+    hipLaunchKernelGGL(plus ? k_low_key_md<true> : k_low_key_md<false>,
+                       dim3(n_items * 16 * (l1 - l0)), dim3(TPB), 0, c->stream, a,
                        md, conv, pmod, l0, n_items, c->d_mods, (const double2 *)c->d_tw_fp,
                        (const double2 *)c->d_rinv_fp);
     LAUNCH_CHECK();
@@ -4416,7 +4436,7 @@ void launch_key_inner_jobs(ckks_context *c, const Strided &ext, const Strided &a
 // i.e. the automorphism is applied on the output side, so each thread reads
 // the extended digits (and c0) at its own index s once for all babies.  With
 // c0 given, acc_b,0[t] += P c0[s] on the Q limbs (the extended lift).
-// grid (N / 256, E); up to kMultiItems items per launch.  At N = 2^16 the
+// grid (N / 256, E); up to multi_items items per launch.  At N = 2^16 the
 // 16 blocks of a tile of 16 rows (4096 positions, which the automorphisms
 // map onto one tile) share blockIdx.x % 8, so they run on one XCD and the
 // permuted stores of the tile fill whole lines in one L2.  Limbs whose prime
@@ -4425,11 +4445,17 @@ void launch_key_inner_jobs(ckks_context *c, const Strided &ext, const Strided &a
 // canonical; the same words).
 // ===========================================================================
 
-template <int MD>
+// MD digits (exactly: no branch between a thread's products; 8 with EXACT
+// false: up to 8) and up to IT items, whose key words are read once.  The
+// stores of the babies and the key reads bound it: 16 ciphertexts of 25
+// limbs, 3 digits, 7 babies, 4 x 350 us with 4 items and 2 x 568 us with 8
+// (4.0 TB/s of stores and key words).
+template <int MD, int IT, bool EXACT>
 __global__ __launch_bounds__(TPB) void k_key_inner_multi(
     Strided ext, int n_items, MultiKeys mk, int n_babies, Batch c0, const u64 *__restrict__ pmod,
-    const u64 *const *__restrict__ outp, int digits, int E, int q_limbs, int L, int K, int logN,
+    const u64 *const *__restrict__ outp, int n_digits, int E, int q_limbs, int L, int K, int logN,
     const ModQ *__restrict__ mods, const double2 *__restrict__ rinv) {
+  const int digits = EXACT ? MD : n_digits;
   int s = blockIdx.x * TPB + threadIdx.x;
   if (logN == 16) {
     const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
@@ -4439,11 +4465,11 @@ __global__ __launch_bounds__(TPB) void k_key_inner_multi(
   const int p = prime_of(l, q_limbs, L);
   const ModQ M = mods[p];
   const size_t N = (size_t)1 << logN;
-  u64 x[kMultiItems][MD];
-  u64 pc[kMultiItems];
+  u64 x[IT][MD];
+  u64 pc[IT];
   const bool lift = l < q_limbs;
 #pragma unroll
-  for (int it = 0; it < kMultiItems; it++) {
+  for (int it = 0; it < IT; it++) {
     if (it < n_items) {
       const u64 *e = ext.base + (size_t)it * ext.stride;
 #pragma unroll
@@ -4457,9 +4483,9 @@ __global__ __launch_bounds__(TPB) void k_key_inner_multi(
   if (M.q < kFpPrimeBound) {
     const double q = (double)M.q, qinv = 1.0 / q;
     const double2 ri = rinv[p];
-    double xd[kMultiItems][MD];
+    double xd[IT][MD];
 #pragma unroll
-    for (int it = 0; it < kMultiItems; it++)
+    for (int it = 0; it < IT; it++)
 #pragma unroll
       for (int j = 0; j < MD; j++)
         xd[it][j] = it < n_items && j < digits ? u52_to_dbl(x[it][j]) : 0.0;
@@ -4496,7 +4522,7 @@ __global__ __launch_bounds__(TPB) void k_key_inner_multi(
         }
       }
 #pragma unroll
-      for (int it = 0; it < kMultiItems; it++) {
+      for (int it = 0; it < IT; it++) {
         if (it < n_items) {
           // |sum| < 1.5 q digits < 2^49
           double a0 = 0.0, a1 = 0.0;
@@ -4520,9 +4546,9 @@ __global__ __launch_bounds__(TPB) void k_key_inner_multi(
   // primes of 2^45 or more: the extended words split once into 30-bit halves
   // for every baby's products, each output's sum of at most MD <= 16
   // products kept as 30-bit half sums (mac30) and reduced once
-  Half30 xh[kMultiItems][MD];
+  Half30 xh[IT][MD];
 #pragma unroll
-  for (int it = 0; it < kMultiItems; it++)
+  for (int it = 0; it < IT; it++)
 #pragma unroll
     for (int j = 0; j < MD; j++)
       xh[it][j] = it < n_items && j < digits ? half30(x[it][j]) : Half30{0, 0};
@@ -4539,7 +4565,7 @@ __global__ __launch_bounds__(TPB) void k_key_inner_multi(
       }
     }
 #pragma unroll
-    for (int it = 0; it < kMultiItems; it++) {
+    for (int it = 0; it < IT; it++) {
       if (it < n_items) {
         Sum30 s0{0, 0, 0, 0}, s1{0, 0, 0, 0};
 #pragma unroll
@@ -4569,7 +4595,8 @@ void launch_key_inner_multi(ckks_context *c, const u64 *ext, size_t ext_stride, 
                               2.0 * n_items * keys.size()),
             2.0 * c->N * E * digits * (double)keys.size() * n_items);
   audit_keyswitch(c, n_items, (int)keys.size(), q_limbs, digits, E);
-  if (n_items < 1 || n_items > kMultiItems) throw std::invalid_argument("key_inner_multi: items");
+  if (n_items < 1 || n_items > multi_items(digits))
+    throw std::invalid_argument("key_inner_multi: items");
   const int nb = (int)keys.size();
   if (nb < 1 || nb > kMaxBatch) throw std::invalid_argument("key_inner_multi: babies");
   MultiKeys mk{};
@@ -4578,16 +4605,14 @@ void launch_key_inner_multi(ckks_context *c, const u64 *ext, size_t ext_stride, 
     mk.ginv[b] = galois_inv[b];
   }
   dim3 grid(c->N / TPB, E);
-  if (digits <= 4)
-    hipLaunchKernelGGL(k_key_inner_multi<4>, grid, dim3(TPB), 0, c->stream,
-                       Strided{(u64 *)ext, ext_stride}, n_items, mk, nb, c0, c->d_pmod, d_outp,
-                       digits, E, q_limbs, c->L, c->K, c->logN, c->d_mods,
-                       (const double2 *)c->d_rinv_fp);
-  else
-    hipLaunchKernelGGL(k_key_inner_multi<kMaxDigits>, grid, dim3(TPB), 0, c->stream,
-                       Strided{(u64 *)ext, ext_stride}, n_items, mk, nb, c0, c->d_pmod, d_outp,
-                       digits, E, q_limbs, c->L, c->K, c->logN, c->d_mods,
-                       (const double2 *)c->d_rinv_fp);
+  auto kern = digits == 1   ? k_key_inner_multi<1, multi_items(1), true>
+              : digits == 2 ? k_key_inner_multi<2, multi_items(2), true>
+              : digits == 3 ? k_key_inner_multi<3, multi_items(3), true>
+              : digits == 4 ? k_key_inner_multi<4, multi_items(4), true>
+                            : k_key_inner_multi<kMaxDigits, multi_items(kMaxDigits), false>;
+  hipLaunchKernelGGL(kern, grid, dim3(TPB), 0, c->stream, Strided{(u64 *)ext, ext_stride}, n_items,
+                     mk, nb, c0, c->d_pmod, d_outp, digits, E, q_limbs, c->L, c->K, c->logN,
+                     c->d_mods, (const double2 *)c->d_rinv_fp);
   LAUNCH_CHECK();
 }
 
@@ -4860,11 +4885,18 @@ __device__ __forceinline__ void mac_table_block(int nz, int logN, int &kb, int &
 // block's ciphertexts at once, the 64-bit path kMacCts at a time; GT >= G
 // groups compiled and a baby step's loads issued one step ahead of its
 // products.  grid (N / 256 x 2 x input groups, E)
+// Babies of id_mask are the ciphertexts themselves (rotation 0), read from
+// cts and lifted by P here instead of being written as extended objects (11
+// us a ciphertext of 25 limbs, and its read): bit b set, baby b of ciphertext
+// i is (P c0, P c1) on the Q limbs, 0 on the special ones.  They are summed
+// before the others: a branch on the kind inside the pipelined loop cost half
+// of its time again.
 template <int GT>
 __global__ __launch_bounds__(TPB) void k_mac_many(const u64 *__restrict__ bab, int n, Batch pts,
                                                   int B, int G, u64 *__restrict__ out, int E,
                                                   int q_limbs, int L, int logN,
-                                                  const ModQ *__restrict__ mods) {
+                                                  const ModQ *__restrict__ mods, Batch cts,
+                                                  u64 id_mask, const u64 *__restrict__ pmod) {
   int kb, z;
   mac_table_block(2 * ((n + kMacCtsFp - 1) / kMacCtsFp), logN, kb, z);
   const int k = kb * TPB + threadIdx.x;
@@ -4872,7 +4904,13 @@ __global__ __launch_bounds__(TPB) void k_mac_many(const u64 *__restrict__ bab, i
   const size_t N = (size_t)1 << logN, EP = 2 * (size_t)E * N;
   const ModQ M = mods[prime_of(l, q_limbs, L)];
   const size_t off = ((size_t)comp * E + l) * N + k;
-  if (M.q < ((u64)1 << 45) && B <= 64) {
+  const bool lift = l < q_limbs;
+  const size_t id_off = ((size_t)comp * q_limbs + l) * N + k;
+  const u64 pm = lift ? pmod[2 * l] : 0, pms = lift ? pmod[2 * l + 1] : 0;
+  // the babies to read (B <= 64), and the ciphertexts' own, taken first
+  const u64 all = B >= 64 ? ~0ull : ((u64)1 << B) - 1;
+  const u64 own = lift ? id_mask & all : 0, read = all & ~id_mask;
+  if (M.q < ((u64)1 << 45)) {
     constexpr int IC = kMacCtsFp;
     const double q = (double)M.q, qinv = 1.0 / q;
     const size_t poff = (size_t)l * N + k;
@@ -4882,22 +4920,7 @@ __global__ __launch_bounds__(TPB) void k_mac_many(const u64 *__restrict__ bab, i
       for (int g = 0; g < GT; g++)
 #pragma unroll
         for (int c = 0; c < IC; c++) acc[g][c] = 0.0;
-      u64 xw[IC], ww[GT];
-      auto issue = [&](int b) {
-#pragma unroll
-        for (int c = 0; c < IC; c++) xw[c] = bab[((size_t)b * n + min(i0 + c, n - 1)) * EP + off];
-#pragma unroll
-        for (int g = 0; g < GT; g++) ww[g] = batch_ptr(pts, min(g, G - 1) * B + b)[poff];
-      };
-      issue(0);
-      for (int b = 0; b < B; b++) {
-        u64 xc[IC], wc[GT];
-#pragma unroll
-        for (int c = 0; c < IC; c++) xc[c] = xw[c];
-#pragma unroll
-        for (int g = 0; g < GT; g++) wc[g] = ww[g];
-        if (b + 1 < B) issue(b + 1);  // the next step's words in flight
-        __builtin_amdgcn_sched_barrier(0);
+      auto products = [&](const u64 (&xc)[IC], const u64 (&wc)[GT]) {
         double x[IC];
 #pragma unroll
         for (int c = 0; c < IC; c++) x[c] = u52_to_dbl(xc[c]);
@@ -4908,6 +4931,36 @@ __global__ __launch_bounds__(TPB) void k_mac_many(const u64 *__restrict__ bab, i
 #pragma unroll
           for (int c = 0; c < IC; c++) acc[g][c] = __dadd_rn(acc[g][c], fp_mulmod(x[c], w, wq, q));
         }
+      };
+      u64 xw[IC], ww[GT];
+      auto plain = [&](int b) {
+#pragma unroll
+        for (int g = 0; g < GT; g++) ww[g] = batch_ptr(pts, min(g, G - 1) * B + b)[poff];
+      };
+      auto issue = [&](int b) {
+#pragma unroll
+        for (int c = 0; c < IC; c++) xw[c] = bab[((size_t)b * n + min(i0 + c, n - 1)) * EP + off];
+        plain(b);
+      };
+      for (u64 m = own; m; m &= m - 1) {
+        plain(__builtin_ctzll(m));
+#pragma unroll
+        for (int c = 0; c < IC; c++) xw[c] = batch_ptr(cts, min(i0 + c, n - 1))[id_off];
+#pragma unroll
+        for (int c = 0; c < IC; c++) xw[c] = shoup_mul(xw[c], pm, pms, M.q);
+        products(xw, ww);
+      }
+      if (read) issue(__builtin_ctzll(read));
+      for (u64 m = read; m;) {
+        u64 xc[IC], wc[GT];
+#pragma unroll
+        for (int c = 0; c < IC; c++) xc[c] = xw[c];
+#pragma unroll
+        for (int g = 0; g < GT; g++) wc[g] = ww[g];
+        m &= m - 1;
+        if (m) issue(__builtin_ctzll(m));  // the next step's words in flight
+        __builtin_amdgcn_sched_barrier(0);
+        products(xc, wc);
       }
 #pragma unroll
       for (int g = 0; g < GT; g++)
@@ -4930,24 +4983,23 @@ __global__ __launch_bounds__(TPB) void k_mac_many(const u64 *__restrict__ bab, i
         acc[g][c] = 0;
         sum[g][c] = Sum30{0, 0, 0, 0};
       }
-    // a baby step's words issued together, one step ahead of their products
-    u64 xw[IC], ww[GT];
-    auto issue = [&](int b) {
+    int terms = 0;
+    auto fold = [&] {
 #pragma unroll
-      for (int c = 0; c < IC; c++) xw[c] = bab[((size_t)b * n + min(i0 + c, n - 1)) * EP + off];
+      for (int g = 0; g < GT; g++)
 #pragma unroll
-      for (int g = 0; g < GT; g++) ww[g] = batch_ptr(pts, min(g, G - 1) * B + b)[(size_t)l * N + k];
+        for (int c = 0; c < IC; c++) {
+          u64 hi, lo;
+          sum30_wide(sum[g][c], hi, lo);
+          acc[g][c] = add_mod(acc[g][c], redc(hi, lo, M.q, M.qinv), M.q);
+          sum[g][c] = Sum30{0, 0, 0, 0};
+        }
+      terms = 0;
     };
-    issue(0);
-    for (int b = 0; b < B; b++) {
-      u64 xc[IC], wc[GT];
-#pragma unroll
-      for (int c = 0; c < IC; c++) xc[c] = xw[c];
-#pragma unroll
-      for (int g = 0; g < GT; g++) wc[g] = ww[g];
-      if (b + 1 < B) issue(b + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      // 16 babies' products as 30-bit half sums (mac30), then reduced
+    // 16 babies' products as 30-bit half sums (mac30), then reduced
+    auto products = [&](const u64 (&xc)[IC], const u64 (&wc)[GT]) {
+      if (terms == 16) fold();
+      terms++;
       Half30 xh[IC];
 #pragma unroll
       for (int c = 0; c < IC; c++) xh[c] = half30(xc[c]);
@@ -4957,18 +5009,39 @@ __global__ __launch_bounds__(TPB) void k_mac_many(const u64 *__restrict__ bab, i
 #pragma unroll
         for (int c = 0; c < IC; c++) mac30(sum[g][c], xh[c], wh);
       }
-      if ((b & 15) == 15 || b == B - 1) {
+    };
+    // a baby step's words issued together, one step ahead of their products
+    u64 xw[IC], ww[GT];
+    auto plain = [&](int b) {
 #pragma unroll
-        for (int g = 0; g < GT; g++)
+      for (int g = 0; g < GT; g++) ww[g] = batch_ptr(pts, min(g, G - 1) * B + b)[(size_t)l * N + k];
+    };
+    auto issue = [&](int b) {
 #pragma unroll
-          for (int c = 0; c < IC; c++) {
-            u64 hi, lo;
-            sum30_wide(sum[g][c], hi, lo);
-            acc[g][c] = add_mod(acc[g][c], redc(hi, lo, M.q, M.qinv), M.q);
-            sum[g][c] = Sum30{0, 0, 0, 0};
-          }
-      }
+      for (int c = 0; c < IC; c++) xw[c] = bab[((size_t)b * n + min(i0 + c, n - 1)) * EP + off];
+      plain(b);
+    };
+    for (u64 m = own; m; m &= m - 1) {
+      plain(__builtin_ctzll(m));
+#pragma unroll
+      for (int c = 0; c < IC; c++) xw[c] = batch_ptr(cts, min(i0 + c, n - 1))[id_off];
+#pragma unroll
+      for (int c = 0; c < IC; c++) xw[c] = shoup_mul(xw[c], pm, pms, M.q);
+      products(xw, ww);
     }
+    if (read) issue(__builtin_ctzll(read));
+    for (u64 m = read; m;) {
+      u64 xc[IC], wc[GT];
+#pragma unroll
+      for (int c = 0; c < IC; c++) xc[c] = xw[c];
+#pragma unroll
+      for (int g = 0; g < GT; g++) wc[g] = ww[g];
+      m &= m - 1;
+      if (m) issue(__builtin_ctzll(m));
+      __builtin_amdgcn_sched_barrier(0);
+      products(xc, wc);
+    }
+    fold();
 #pragma unroll
     for (int g = 0; g < GT; g++)
 #pragma unroll
@@ -4978,7 +5051,7 @@ __global__ __launch_bounds__(TPB) void k_mac_many(const u64 *__restrict__ bab, i
 }
 
 void launch_mac_many(ckks_context *c, const u64 *bab, int n, const Batch &pts, int B, int G,
-                     u64 *out, int E, int q_limbs) {
+                     u64 *out, int E, int q_limbs, const Batch &cts, u64 id_mask) {
   KTimer kt(c, "mac_many", 8.0 * c->N * E * (2.0 * n * B + (double)G * B + 2.0 * G * n),
             2.0 * c->N * E * (double)n * B * G);
   audit_pt(c, (double)G * B * E);
@@ -4986,7 +5059,8 @@ void launch_mac_many(ckks_context *c, const u64 *bab, int n, const Batch &pts, i
     throw std::invalid_argument("mac_many: 1 <= groups <= 2 and groups x babies <= 64");
   dim3 grid(c->N / TPB * 2 * ((n + kMacCtsFp - 1) / kMacCtsFp), E);
   hipLaunchKernelGGL(G <= 1 ? k_mac_many<1> : k_mac_many<kMacGroups>, grid, dim3(TPB), 0,
-                     c->stream, bab, n, pts, B, G, out, E, q_limbs, c->L, c->logN, c->d_mods);
+                     c->stream, bab, n, pts, B, G, out, E, q_limbs, c->L, c->logN, c->d_mods, cts,
+                     id_mask, c->d_pmod);
   LAUNCH_CHECK();
 }
 

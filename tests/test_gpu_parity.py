@@ -804,6 +804,62 @@ def test_keyswitch_small_batches_full_size(params, levels):
     ctx.close()
 
 
+@pytest.mark.slow
+@pytest.mark.parametrize("params", [
+    "keyswitch",
+    dict(log_n=16, depth=9, dnum=2, dcrt_bits=59, first_mod=60, special_bits=60),
+    dict(log_n=15, depth=5, dnum=3, dcrt_bits=40, first_mod=60, special_bits=60),
+])
+def test_giant_chain_adds_in_the_moddown(params):
+    """The giant Horner chains, whose sums are taken in the rotations'
+    ModDown, give the words of rotations and additions: batches on one and on
+    several streams, extended babies with the ciphertext itself among them (in
+    one pass for all ciphertexts or one by one)."""
+    fhe = _fhe()
+    B, G, giant, limbs = 3, 3, 8, 6
+    client, ctx = device_context(params, rotations=(1, 2, giant))
+    rng = np.random.default_rng(31)
+    slots, n = 32, 17
+    cts = [client.encrypt(rng.uniform(-1, 1, slots), slots=slots, cur_limbs=limbs, enc_id=700 + i)
+           for i in range(n)]
+    rows = rng.uniform(-1, 1, (B * G, slots))
+    for ext in (False, True):
+        pts = fhe.encode_rows(ctx, rows, limbs=limbs, scale=ctx.scale_at(limbs), slots=slots,
+                              is_ext=ext)
+        offsets = [0, 1, 2]
+        if ext:
+            def run(c, p, g):
+                return fhe.hoisted_mac_sum_ext_many(c, offsets, p, giant, g, ctx)
+        else:
+            babies = [fhe.prepare_hoisted_baby_rotations(c, offsets, ctx) for c in cts]
+
+            def run(c, p, g):
+                return fhe.hoisted_mac_sum_many(babies[: len(c)], p, giant, g, ctx)
+        want = None
+        for g in reversed(range(G)):
+            inner = run(cts, pts[g * B: (g + 1) * B], 1)
+            if ext:
+                for i in (0, 8, 16):
+                    one = fhe.hoisted_mac_sum_ext_many(cts[i: i + 1], offsets,
+                                                       pts[g * B: (g + 1) * B], giant, 1, ctx)
+                    assert np.array_equal(one[0].download(), inner[i].download()), (g, i)
+            if want is None:
+                want = inner
+            else:
+                want = fhe.homo_add_many(fhe.homo_rotate_many(want, giant, ctx), inner, ctx)
+        words = [w.download() for w in want]
+        for k in (1, 3, n):
+            got = run(cts[:k], pts, G)
+            for i in range(k):
+                assert np.array_equal(got[i].download(), words[i]), (ext, k, i)
+    one = fhe.hoisted_mac_sum(cts[0], offsets, fhe.encode_rows(
+        ctx, rows, limbs=limbs, scale=ctx.scale_at(limbs), slots=slots), giant, G, ctx)
+    first = fhe.hoisted_mac_sum_many(babies[:1], fhe.encode_rows(
+        ctx, rows, limbs=limbs, scale=ctx.scale_at(limbs), slots=slots), giant, G, ctx)
+    assert np.array_equal(one.download(), first[0].download())
+    ctx.close()
+
+
 def test_linear_combination_matches_composed_ops():
     """One fused launch = mul_scalar + add + add_scalar on the same words,
     with terms holding more limbs than the output."""
