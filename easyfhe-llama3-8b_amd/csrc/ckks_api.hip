@@ -746,9 +746,8 @@ static void build_context(ckks_context *c, const ckks_params &p) {
 // stream is drained and the buffers too small for the request are dropped.
 static constexpr size_t kStageUnit = (size_t)1 << 20, kStageCap = (size_t)1 << 30;
 
-namespace ckks {
-void upload_async(ckks_context *c, void *dst, const void *src, size_t bytes) {
-  if (bytes == 0) return;
+// A staging buffer of at least `bytes` whose last copy has completed.
+static ckks_context::StageBuf *stage_buffer(ckks_context *c, size_t bytes) {
   ckks_context::StageBuf *pick = nullptr;
   for (auto &b : c->stage) {
     if (b.bytes < bytes) continue;
@@ -788,6 +787,13 @@ void upload_async(ckks_context *c, void *dst, const void *src, size_t bytes) {
       pick = &c->stage.back();
     }
   }
+  return pick;
+}
+
+namespace ckks {
+void upload_async(ckks_context *c, void *dst, const void *src, size_t bytes) {
+  if (bytes == 0) return;
+  ckks_context::StageBuf *pick = stage_buffer(c, bytes);
   memcpy(pick->p, src, bytes);
   HIPCHECK(hipMemcpyAsync(dst, pick->p, bytes, hipMemcpyHostToDevice, c->stream));
   HIPCHECK(hipEventRecord(pick->ev, c->stream));
@@ -1997,14 +2003,11 @@ int ckks_encrypt(ckks_context *c, const double *re, const double *im, int slots,
   ckks_ct *ct = new_ct(c, 2, limbs, 0, slots, scale, 1);
   Scratch s(c);
   double *dre = (double *)s.get(slots), *dim = im ? (double *)s.get(slots) : nullptr;
-  HIPCHECK(hipMemcpyAsync(dre, re, sizeof(double) * slots, hipMemcpyHostToDevice, c->stream));
-  if (im)
-    HIPCHECK(hipMemcpyAsync(dim, im, sizeof(double) * slots, hipMemcpyHostToDevice, c->stream));
-  Batch o{};
-  o.p[0] = ct->d;
-  launch_encode(c, dre, dim, 1, slots, scale, limbs, 0, o);
-  launch_encrypt_finish(c, ct->d, limbs, enc_id);
-  HIPCHECK(hipStreamSynchronize(c->stream));  // host buffers are the caller's
+  // through pinned staging: the caller's buffers are free on return, and the
+  // next call's host work runs beside this one's kernels
+  upload_async(c, dre, re, sizeof(double) * slots);
+  if (im) upload_async(c, dim, im, sizeof(double) * slots);
+  launch_encrypt(c, dre, dim, slots, scale, ct->d, limbs, enc_id);
   *out = ct;
   API_END
 }
@@ -2016,12 +2019,15 @@ int ckks_decrypt(ckks_context *c, const ckks_ct *ct, double *re, double *im) {
   require(ct->polys >= 1 && !ct->is_ext, "decrypt needs a Q-basis ciphertext");
   fft_table(c, ct->slots);
   Scratch s(c);
-  double *dre = (double *)s.get(ct->slots), *dim = (double *)s.get(ct->slots);
+  // both parts in one copy, through pinned staging
+  const size_t part = sizeof(double) * ct->slots, bytes = (im ? 2 : 1) * part;
+  double *dre = (double *)s.get(2 * (size_t)ct->slots), *dim = dre + ct->slots;
   launch_decrypt_decode(c, ct, dre, dim);
-  HIPCHECK(hipMemcpyAsync(re, dre, sizeof(double) * ct->slots, hipMemcpyDeviceToHost, c->stream));
-  if (im)
-    HIPCHECK(hipMemcpyAsync(im, dim, sizeof(double) * ct->slots, hipMemcpyDeviceToHost, c->stream));
+  ckks_context::StageBuf *b = stage_buffer(c, bytes);
+  HIPCHECK(hipMemcpyAsync(b->p, dre, bytes, hipMemcpyDeviceToHost, c->stream));
   HIPCHECK(hipStreamSynchronize(c->stream));
+  memcpy(re, b->p, part);
+  if (im) memcpy(im, (const char *)b->p + part, part);
   API_END
 }
 

@@ -667,8 +667,10 @@ void launch_keygen(ckks_context *c, DeviceKey &key, u64 id, int relin, u64 galoi
 // residues of a signed integer polynomial e[N] over `limbs` limbs, then NTT
 void launch_expand_ntt(ckks_context *c, const long long *e, u64 *out, int limbs, int q_limbs);
 void launch_encode(ckks_context *c, const double *d_re, const double *d_im, int rows,
-                   int slots, double scale, int limbs, int is_ext, const Batch &out);
-void launch_encrypt_finish(ckks_context *c, u64 *ct, int limbs, u32 enc_id);
+                   int slots, double scale, int limbs, int is_ext, const Batch &out,
+                   const long long *e = nullptr);
+void launch_encrypt(ckks_context *c, const double *d_re, const double *d_im, int slots,
+                    double scale, u64 *ct, int limbs, u32 enc_id);
 void launch_decrypt_decode(ckks_context *c, const ckks_ct *ct, double *d_re, double *d_im);
 void launch_scalar_encode(ckks_context *c, double v, int limbs, u64 *out);
 // operations per second of the register-only probe (blocks x 256 threads,

@@ -5606,9 +5606,8 @@ void launch_keygen(ckks_context *c, DeviceKey &key, u64 id, int relin, u64 galoi
 }
 
 // Encryption: c1 = uniform (ENC_A, id, l) in the NTT domain,
-// c0 = e - c1 s + m, with m already encoded in c0.  grid (N / 4 / 256, limbs)
-__global__ void k_encrypt(u64 seed, u32 id, const u64 *__restrict__ e_ntt,
-                          const u64 *__restrict__ s_ntt, u64 *__restrict__ ct, int limbs,
+// c0 = m + e - c1 s, with m + e already in c0.  grid (N / 4 / 256, limbs)
+__global__ void k_encrypt(u64 seed, u32 id, const u64 *__restrict__ s_ntt, u64 *__restrict__ ct, int limbs,
                           int logN, const ModQ *__restrict__ mods) {
   const int t = blockIdx.x * TPB + threadIdx.x;
   const int l = blockIdx.y;
@@ -5626,28 +5625,27 @@ __global__ void k_encrypt(u64 seed, u32 id, const u64 *__restrict__ e_ntt,
     const u64 hi = (u64)blk[4 * r + 2] | ((u64)blk[4 * r + 3] << 32);
     const u64 a = wide_mod(hi, lo, M);
     c1[k] = a;
-    c0[k] = add_mod(sub_mod(e_ntt[l * N + k], mul_mod(a, s_ntt[l * N + k], M), M.q), c0[k], M.q);
+    c0[k] = sub_mod(c0[k], mul_mod(a, s_ntt[l * N + k], M), M.q);
   }
 }
 
-void launch_encrypt_finish(ckks_context *c, u64 *ct, int limbs, u32 enc_id) {
+// The message and the error are transformed together: the transform is linear
+// and its words canonical, so one NTT gives the words of two (36 limbs of
+// N = 2^16: 146 us of kernels a ciphertext in 11 launches, now 89 in 8).
+void launch_encrypt(ckks_context *c, const double *d_re, const double *d_im, int slots,
+                    double scale, u64 *ct, int limbs, u32 enc_id) {
   const int N = c->N;
   long long *e = (long long *)c->pool.alloc(sizeof(long long) * N);
-  u64 *en = (u64 *)c->pool.alloc(sizeof(u64) * (size_t)limbs * N);
   hipLaunchKernelGGL(k_sample_cbd, dim3((N / 8 + TPB - 1) / TPB), dim3(TPB), 0, c->stream,
                      c->params.seed, (u32)DOM_ENC_E, enc_id, 0u, e, N);
   LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_expand_int, dim3(N / TPB, limbs), dim3(TPB), 0, c->stream, e, en,
-                     c->logN, limbs, c->L, c->d_mods);
-  LAUNCH_CHECK();
-  Batch b{};
-  b.p[0] = en;
-  launch_ntt(c, b, b, 1, 0, limbs, limbs, false);
+  Batch o{};
+  o.p[0] = ct;
+  launch_encode(c, d_re, d_im, 1, slots, scale, limbs, 0, o, e);
   hipLaunchKernelGGL(k_encrypt, dim3((N / 4 + TPB - 1) / TPB, limbs), dim3(TPB), 0, c->stream,
-                     c->params.seed, enc_id, en, c->d_secret, ct, limbs, c->logN, c->d_mods);
+                     c->params.seed, enc_id, c->d_secret, ct, limbs, c->logN, c->d_mods);
   LAUNCH_CHECK();
   c->pool.release(e, sizeof(long long) * N);
-  c->pool.release(en, sizeof(u64) * (size_t)limbs * N);
 }
 
 // ===========================================================================
@@ -5689,7 +5687,7 @@ __global__ void k_fft_place(const double *__restrict__ re, const double *__restr
 // so every rounding, is that of the stage-by-stage definition above.
 constexpr int kFftTile = 2048;
 
-// grid (n / tile, rows), tile = min(n, kFftTile)
+// rows of fewer than kFftTile points: tile = n, grid (1, rows)
 __global__ __launch_bounds__(TPB) void k_fft_tile(cplx *__restrict__ x, int n, int tile,
                                                   const cplx *__restrict__ tw) {
   __shared__ cplx sm[kFftTile];
@@ -5709,6 +5707,50 @@ __global__ __launch_bounds__(TPB) void k_fft_tile(cplx *__restrict__ x, int n, i
     __syncthreads();
   }
   for (int i = threadIdx.x; i < tile; i += TPB) row[i] = sm[i];
+}
+
+// k_fft_tile for whole tiles: 8 points a thread in registers, three stages
+// between exchanges (the word positions of Ring), the same operations on the
+// same operands.  A barrier and a twiddle wait after each of 11 stages held
+// the few blocks of a row: one row of 32768 points 15.5 -> 5.6 us.
+// grid (n / kFftTile, rows)
+template <int RI>
+__device__ __forceinline__ void fft_rounds(cplx (&x)[8], cplx *__restrict__ sm, int n,
+                                           const cplx *__restrict__ tw, int t) {
+  using G = Ring<11, 3>;
+  constexpr int win = G::iwin(RI), s0 = G::ilo(RI) - win, s1 = G::ihi(RI) - win;
+  cplx w[7];
+#pragma unroll
+  for (int i = s0; i < s1; i++)
+#pragma unroll
+    for (int m = 0; m < (1 << i); m++)
+      w[(1 << i) - 1 + m] = tw[((m << win) | (t & ((1 << win) - 1))) * (n >> (win + i + 1))];
+  if constexpr (RI == 0) ring_exchange<11, 3>(x, sm, 8, win, t);
+  else ring_exchange<11, 3>(x, sm, G::iwin(RI - 1), win, t);
+#pragma unroll
+  for (int i = s0; i < s1; i++)
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      if (k & (1 << i)) continue;
+      const cplx u = x[k], v = cmul(x[k + (1 << i)], w[(1 << i) - 1 + (k & ((1 << i) - 1))]);
+      x[k] = cplx{__dadd_rn(u.re, v.re), __dadd_rn(u.im, v.im)};
+      x[k + (1 << i)] = cplx{__dsub_rn(u.re, v.re), __dsub_rn(u.im, v.im)};
+    }
+  if constexpr (RI + 1 < G::R) fft_rounds<RI + 1>(x, sm, n, tw, t);
+}
+
+__global__ __launch_bounds__(TPB) void k_fft_tile8(cplx *__restrict__ x, int n,
+                                                   const cplx *__restrict__ tw) {
+  static_assert(kFftTile == 2048 && TPB == 256, "8 points a thread");
+  __shared__ cplx sm[Ring<11, 3>::kLds];
+  cplx *row = x + (size_t)blockIdx.y * n + (size_t)blockIdx.x * kFftTile;
+  const int t = threadIdx.x;
+  cplx v[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) v[k] = row[t + 256 * k];
+  fft_rounds<0>(v, sm, n, tw, t);
+#pragma unroll
+  for (int k = 0; k < 8; k++) row[t + 256 * k] = v[k];
 }
 
 // grid (kFftTile / 256, rows); n = M kFftTile
@@ -5743,7 +5785,10 @@ static void launch_fft(ckks_context *c, cplx *x, int rows, int n, const cplx *tw
   if (n < 2 || rows < 1) return;
   if (rows > 65535) throw std::invalid_argument("fft: at most 65535 rows per launch");
   const int tile = n < kFftTile ? n : kFftTile;
-  hipLaunchKernelGGL(k_fft_tile, dim3(n / tile, rows), dim3(TPB), 0, c->stream, x, n, tile, tw);
+  if (tile == kFftTile)
+    hipLaunchKernelGGL(k_fft_tile8, dim3(n / tile, rows), dim3(TPB), 0, c->stream, x, n, tw);
+  else
+    hipLaunchKernelGGL(k_fft_tile, dim3(1, rows), dim3(TPB), 0, c->stream, x, n, tile, tw);
   LAUNCH_CHECK();
   const dim3 g(kFftTile / TPB, rows);
   switch (n / tile) {
@@ -5771,10 +5816,15 @@ __device__ u64 dbl_residue(double v, const ModQ &M) {
 
 // Encoder tail: u = (x_k / n) * twist_k, coefficient k gap and (k + n) gap
 // get rint(scale u.re), rint(scale u.im); then residues for every limb, the
-// rounded value formed once per coefficient.  grid (N / 256, rows)
+// rounded value formed once per coefficient and block.  With e (encryption),
+// the error's residue is added: its transform is then the message's.  A block
+// takes `per` limbs: one row of 36 limbs is 256 blocks of N / 256
+// coefficients, a serial chain of limbs on one wave a SIMD (19 us), so few
+// rows are split over the limbs (11 us with the error's residues).  grid (N / 256, rows, limb parts)
 __global__ void k_encode_finish(const cplx *__restrict__ x, const cplx *__restrict__ twist,
-                                Batch out, int n, int logN, double scale, int total, int q_limbs,
-                                int L, const ModQ *__restrict__ mods) {
+                                Batch out, int n, int logN, double scale, int total, int per,
+                                int q_limbs, int L, const ModQ *__restrict__ mods,
+                                const long long *__restrict__ e) {
   const int k = blockIdx.x * TPB + threadIdx.x;  // coefficient index
   const int N = 1 << logN, gap = N / (2 * n);
   double v = 0.0;
@@ -5787,28 +5837,39 @@ __global__ void k_encode_finish(const cplx *__restrict__ x, const cplx *__restri
     u = cmul(u, twist[kk]);
     v = rint(__dmul_rn(scale, idx < n ? u.re : u.im));
   }
+  const long long ek = e ? e[k] : 0;
   u64 *o = batch_ptr(out, blockIdx.y) + k;
-  for (int l = 0; l < total; l++)
-    o[(size_t)l << logN] = dbl_residue(v, mods[prime_of(l, q_limbs, L)]);
+  const int l0 = blockIdx.z * per, l1 = min(l0 + per, total);
+  for (int l = l0; l < l1; l++) {
+    const ModQ M = mods[prime_of(l, q_limbs, L)];
+    u64 r = dbl_residue(v, M);
+    if (e) r = add_mod(r, signed_residue(ek, M), M.q);
+    o[(size_t)l << logN] = r;
+  }
 }
 
 // Encoder tail over rows already placed in x ([rows][n], slot j at
-// bit-reversed perm[j]): inverse FFT, twist, rounding, residues, NTT.
+// bit-reversed perm[j]): inverse FFT, twist, rounding, residues (with e, plus
+// the error polynomial's: one row), NTT.
 static void encode_placed(ckks_context *c, cplx *x, int rows, int slots, double scale,
-                          int limbs, int is_ext, const Batch &out) {
+                          int limbs, int is_ext, const Batch &out, const long long *e = nullptr) {
   const FFTTable &t = c->fft.at(slots);
   const int n = slots;
   launch_fft(c, x, rows, n, (const cplx *)t.tw_inv);
   const int total = limbs + (is_ext ? c->alpha : 0);
-  hipLaunchKernelGGL(k_encode_finish, dim3(c->N / TPB, rows), dim3(TPB), 0, c->stream, x,
-                     (const cplx *)t.twist, out, n, c->logN, scale, total, limbs, c->L,
-                     c->d_mods);
+  // about eight blocks a CU
+  const int parts = std::max(1, std::min(total, 8 * kCUs / std::max(1, c->N / TPB * rows)));
+  const int per = (total + parts - 1) / parts;
+  hipLaunchKernelGGL(k_encode_finish, dim3(c->N / TPB, rows, (total + per - 1) / per), dim3(TPB), 0,
+                     c->stream, x, (const cplx *)t.twist, out, n, c->logN, scale, total, per, limbs,
+                     c->L, c->d_mods, e);
   LAUNCH_CHECK();
   launch_ntt(c, out, out, rows, 0, total, limbs, false);
 }
 
 void launch_encode(ckks_context *c, const double *d_re, const double *d_im, int rows,
-                   int slots, double scale, int limbs, int is_ext, const Batch &out) {
+                   int slots, double scale, int limbs, int is_ext, const Batch &out,
+                   const long long *e) {
   const FFTTable &t = c->fft.at(slots);
   const int n = slots;
   int logn = 0;
@@ -5817,7 +5878,7 @@ void launch_encode(ckks_context *c, const double *d_re, const double *d_im, int 
   hipLaunchKernelGGL(k_fft_place, dim3((n + TPB - 1) / TPB, rows), dim3(TPB), 0, c->stream,
                      d_re, d_im, x, t.perm, n, logn);
   LAUNCH_CHECK();
-  encode_placed(c, x, rows, slots, scale, limbs, is_ext, out);
+  encode_placed(c, x, rows, slots, scale, limbs, is_ext, out, e);
   c->pool.release(x, sizeof(cplx) * (size_t)rows * n);
 }
 

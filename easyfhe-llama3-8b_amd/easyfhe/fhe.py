@@ -379,24 +379,29 @@ class Client:
         z = np.asarray(values).reshape(-1)
         if z.size > slots:
             raise ValueError(f"{z.size} values do not fit {slots} slots")
-        buf = np.zeros(slots, dtype=np.complex128)
-        buf[: z.size] = z
-        re = np.ascontiguousarray(buf.real)
-        im = np.ascontiguousarray(buf.imag)
+        if z.dtype.kind not in "biufc":
+            z = z.astype(np.complex128)
+        re = np.zeros(slots)
+        re[: z.size] = z.real
+        im = None  # real values: no imaginary part to upload
+        if z.dtype.kind == "c":
+            im = np.zeros(slots)
+            im[: z.size] = z.imag
         eid = ctx.next_encryption_id() if enc_id is None else int(enc_id)
         out = ctypes.c_void_p()
         check(lib.ckks_encrypt(ctx.handle, re.ctypes.data_as(_native.DP),
-                               im.ctypes.data_as(_native.DP), slots, limbs, scale,
-                               eid & 0xFFFFFFFF, ctypes.byref(out)))
+                               None if im is None else im.ctypes.data_as(_native.DP), slots,
+                               limbs, scale, eid & 0xFFFFFFFF, ctypes.byref(out)))
         return _wrap(ctx, out)
 
     def decrypt_complex(self, ct: Ciphertext) -> np.ndarray:
         slots = ct.slots
-        re = np.zeros(slots)
-        im = np.zeros(slots)
+        re, im = np.empty(slots), np.empty(slots)
         check(lib.ckks_decrypt(self.context.handle, ct.handle, re.ctypes.data_as(_native.DP),
                                im.ctypes.data_as(_native.DP)))
-        return re + 1j * im
+        z = np.empty(slots, dtype=np.complex128)
+        z.real, z.imag = re, im
+        return z
 
     def decrypt(self, ct: Ciphertext) -> np.ndarray:
         """Real part of the decrypted slots (reference backend.py:305-313)."""

@@ -109,6 +109,31 @@ def test_encrypt_decrypt_parity(name):
     assert np.abs(client.decrypt_complex(ct) - zs).max() < 1e-7
 
 
+@pytest.mark.parametrize("slots", [2, 64, 2048])
+def test_encrypt_input_forms(slots):
+    """Real, complex, integer and short inputs, and a buffer overwritten right
+    after the call, give the oracle's limbs; rows below, at and above the
+    register FFT's tile."""
+    fhe = _fhe()
+    client, ctx = device_context("small", relin=False)
+    orc = oracle_context("small")
+    rng = np.random.default_rng(slots)
+    sc = ctx.scale_at(ctx.L)
+    full = rng.uniform(-1, 1, slots)
+    forms = [full, full.astype(np.float32), full + 1j * rng.uniform(-1, 1, slots),
+             (1j * full).astype(np.complex64), np.arange(slots) - 3, list(full[: slots // 2]), full[:1]]
+    for i, z in enumerate(forms):
+        pad = np.zeros(slots, dtype=np.complex128)
+        pad[: len(z)] = z
+        want = orc.encrypt(pad, slots=slots, scale=sc, limbs=ctx.L, enc_id=60 + i)
+        buf = np.array(z)
+        ct = client.encrypt(buf, slots=slots, enc_id=60 + i)
+        buf[:] = 7
+        assert np.array_equal(ct.download(), want), i
+        # noise of a fresh encryption at scale 2^40
+        assert np.abs(client.decrypt_complex(ct) - pad).max() < 1e-6
+
+
 def test_encode_parity_large_scale():
     """Encoder integer path for |coefficients| >= 2^63 (scale 2^80)."""
     fhe = _fhe()
