@@ -446,8 +446,8 @@ static const u64 *relin_rs_table(ckks_context *c, int limbs, int D) {
     for (int j = 0; j < c->alpha; j++) P = mulmod_h(P, c->primes[c->L + j] % q, q);
     return P;
   };
-  // u64 part, then [T][D] (P p_1..p_{j-1} mod q_t, / q_t) as doubles for the
-  // fp64 kernel (targets below 2^45)
+  // u64 part, then [T][D] (P p_1..p_{j-1} mod q_t, / q_t) as doubles for
+  // targets below 2^45, as words with the Shoup constant for the others
   const size_t words = 4 * (size_t)T + 2 * (size_t)T * D + 2 * (size_t)D + 3 * (size_t)D * D;
   std::vector<u64> h(words + 2 * (size_t)T * D, 0);
   u64 *pm = h.data() + 4 * (size_t)T, *pp = pm + (size_t)T * D, *pi = pp + (size_t)T * D;
@@ -458,8 +458,14 @@ static const u64 *relin_rs_table(ckks_context *c, int limbs, int D) {
     u64 prod = 1;  // p_1..p_j mod q
     for (int j = 0; j < D; j++) {
       const u64 f = mulmod_h(P, prod, q);
-      pmf[2 * ((size_t)t * D + j)] = (double)f;
-      pmf[2 * ((size_t)t * D + j) + 1] = (double)f / (double)q;
+      double *e = pmf + 2 * ((size_t)t * D + j);
+      if (c->prime_fp[t]) {
+        e[0] = (double)f;
+        e[1] = (double)f / (double)q;
+      } else {
+        const u64 w[2] = {f, shoup_h(f, q)};
+        memcpy(e, w, sizeof(w));
+      }
       pm[(size_t)t * D + j] = (u64)(((u128)f << 64) % q);
       prod = mulmod_h(prod, p(j) % q, q);
       pp[(size_t)t * D + j] = mulmod_h(P, prod, q);

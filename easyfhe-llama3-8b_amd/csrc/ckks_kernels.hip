@@ -3583,7 +3583,8 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
     }
     if constexpr (RS) {
       if (lifts) {
-        // the lifts, in the lanes of each dropped target (fp64 primes; the
+        // the lifts, in the lanes of each dropped target (whose value is an
+        // fp64 residue or, of a prime of 2^45 or more, the canonical word; the
         // transposed order puts target t in lane group t % 4, row t % 16 / 4)
         const u64 *rpinv = rs + 2 * (size_t)T * RSD;
         const u64 *rchain = rpinv + 2 * RSD;
@@ -3607,7 +3608,8 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
             for (int r = 0; r < 16; r++) {
               // a mask select, so that y keeps static indices
               const u64 msk = 0ull - (u64)ee_d;
-              const u64 yd = fp_canon(as_dbl((y[0][r] & ~msk) | (y[1][r] & msk)), qinv, q);
+              const u64 yr = (y[0][r] & ~msk) | (y[1][r] & msk);
+              const u64 yd = qd < kFpPrimeBound ? fp_canon(as_dbl(yr), qinv, q) : yr;
               u64 u = shoup_mul(sub_mod(xs[4096 * r], yd, qd), pinv, pinvs, qd);
 #pragma unroll
               for (int m = 0; m < j; m++) {
@@ -3645,13 +3647,15 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
               y[ee][r] = dbl_bits(yv);
             }
           } else {
-            const u64 qu = w[0], qinvm = w[1], pmM = w[12 + 4 * j];
+            // y + r_j f (- f p) with f = [P p_1..p_j]_t by its Shoup constant,
+            // lazily: below 2q + 4q with the correction, reduced to below 3q
+            const u64 qu = w[0], f = w[10 + 4 * j], fs = w[11 + 4 * j], neg = qu - w[13 + 4 * j];
+            const LazyQ Q{qu, 0 - qu, (u32)ttw[(size_t)t * 32 + 16], 0, 0};
 #pragma unroll
             for (int r = 0; r < 16; r++) {
               const u64 rj = lift[(j * 16 + r) * 64 + wave * 16 + col];
-              u64 yw = add_mod(y[ee][r], redc(__umul64hi(rj, pmM), rj * pmM, qu, qinvm), qu);
-              if (rj > (qj - 1) / 2) yw = sub_mod(yw, w[13 + 4 * j], qu);
-              y[ee][r] = yw;
+              const u64 yc = y[ee][r] + (rj > (qj - 1) / 2 ? neg : 0);
+              y[ee][r] = lazy_reduce(shoup_add(yc, rj, f, fs, Q), Q);
             }
           }
         }
@@ -3689,7 +3693,7 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
         }
       } else {
         // a prime of 2^45 or more: the forward high pass here, or (flag 4)
-        // stored canonical for the launch after the kernel
+        // stored below 3q for the launch after the kernel
         if (!wide_tgt_out) {
           const u64 qu = w[0];
           LazyQ Q{qu, 0 - qu, (u32)tw0[16], 0, 0};
@@ -3891,9 +3895,12 @@ bool convert_h4_rs_ok(const ckks_context *c, const BCTable &t, int D) {
   if (!(D >= 1 && D <= 2 && t.nd > D && convert_h4_ok(c, t) && convert_h4_lds(t, D) <= 65536 &&
         ((t.nd - 1) >> 3) == ((t.nd - D) >> 3)))
     return false;
-  for (int j = 0; j < D; j++)
-    if (c->primes[t.nd - 1 - j] >= kFpPrimeBound) return false;
-  return true;
+  // fp64 targets add their lifts in fp64, which holds those of dropped primes
+  // below 2^45; wide dropped primes (the 59-bit chain) need wide kept targets
+  bool wide_drop = false, fp_kept = false;
+  for (int j = 0; j < D; j++) wide_drop = wide_drop || !c->prime_fp[t.nd - 1 - j];
+  for (int i = 0; i < t.nd - D; i++) fp_kept = fp_kept || c->prime_fp[i];
+  return !(wide_drop && fp_kept);
 }
 
 void launch_convert_h4_rs(ckks_context *c, const Batch &src, const Batch &dst, int n_items,
