@@ -1737,7 +1737,8 @@ static const u64 *rescale_d_table(ckks_context *c, int limbs, int D) {
 
 // Rescale n ciphertexts of `polys` polynomials each by their last D primes:
 // the inverse NTT of those limbs, the combined lift (k_rescale_lift), its
-// forward NTT and the combine, which at N = 2^16 runs in the NTT's last pass.
+// forward NTT and the combine; at N = 2^16 the lift runs between the NTTs'
+// halves (k_rescale_mid) and the combine in the NTT's last pass.
 // The words equal those of D rescales in a row.
 static void rescale_batch(ckks_context *c, const ckks_ct *const *in, int n, ckks_ct **out,
                           int D = 1) {
@@ -1758,9 +1759,16 @@ static void rescale_batch(ckks_context *c, const ckks_ct *const *in, int n, ckks
         src.p[i * polys + p] = in[b0 + i]->d + (size_t)p * limbs * N;
         dst.p[i * polys + p] = out[b0 + i]->d + (size_t)p * T * N;
       }
-    launch_ntt(c, src, strided(last - (size_t)T * N, (size_t)D * N), items, T, D, limbs, true);
-    launch_rescale_lift(c, strided(last, (size_t)D * N), strided(w, (size_t)T * N), items, limbs,
-                        D, tab);
+    const Batch wb = strided(w, (size_t)T * N), lb = strided(last, (size_t)D * N);
+    const Batch lt = strided(last - (size_t)T * N, (size_t)D * N);  // limb T at last
+    const bool mid = rescale_mid_ok(c, D);
+    if (mid) {
+      launch_ntt_inv_low(c, src, lt, items, T, D, limbs);
+      launch_rescale_mid(c, lb, wb, items, limbs, D, tab);
+    } else {
+      launch_ntt(c, src, lt, items, T, D, limbs, true);
+      launch_rescale_lift(c, lb, wb, items, limbs, D, tab);
+    }
     if (fused) {
       Batch acc{}, o{};
       for (int i = 0; i < nb; i++) {
@@ -1768,11 +1776,12 @@ static void rescale_batch(ckks_context *c, const ckks_ct *const *in, int n, ckks
         o.p[i] = out[b0 + i]->d;
       }
       std::vector<u64> gal(nb, 1);
-      launch_ntt_moddown(c, strided(w, (size_t)T * N), nb, T, acc, limbs, tab, Batch{}, 0,
-                         gal.data(), o, (u64)T * N);
+      launch_ntt_moddown(c, wb, nb, T, acc, limbs, tab, Batch{}, 0, gal.data(), o, (u64)T * N,
+                         nullptr, nullptr, mid);
     } else {
-      launch_ntt(c, strided(w, (size_t)T * N), strided(w, (size_t)T * N), items, 0, T, T, false);
-      launch_rescale_finish(c, src, strided(w, (size_t)T * N), dst, items, T, tab);
+      if (mid) launch_ntt_fwd_low(c, wb, items, 0, T, T);
+      else launch_ntt(c, wb, wb, items, 0, T, T, false);
+      launch_rescale_finish(c, src, wb, dst, items, T, tab);
     }
   }
 }

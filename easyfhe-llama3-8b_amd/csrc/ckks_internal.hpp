@@ -612,6 +612,11 @@ void launch_convert_h4_digits(ckks_context *c, const Batch &src, const Batch &ds
                               const BCTable *const *tabs, int digits, int q_limbs, bool packed);
 void launch_rescale_lift(ckks_context *c, const Batch &last, const Batch &w, int n_items,
                          int limbs, int D, const u64 *tab);
+// N = 2^16, D <= 2 (rescale_mid_ok): launch_rescale_lift of limbs that only went through the inverse low
+// pass, into limbs that only lack the forward low pass
+bool rescale_mid_ok(const ckks_context *c, int D);
+void launch_rescale_mid(ckks_context *c, const Batch &last, const Batch &w, int n_items, int limbs,
+                        int D, const u64 *tab);
 void launch_rescale_finish(ckks_context *c, const Batch &src, const Batch &w, const Batch &out,
                            int n_items, int T, const u64 *inv);
 void launch_bc_down_rescale(ckks_context *c, const Batch &src, const Batch &dst, int n_items,

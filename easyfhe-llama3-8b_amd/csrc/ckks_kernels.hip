@@ -4747,6 +4747,131 @@ void launch_rescale_lift(ckks_context *c, const Batch &last, const Batch &w, int
   LAUNCH_CHECK();
 }
 
+// N = 2^16: k_rescale_lift between the NTT halves, one thread a column (words
+// c + 4096 k): the inverse high pass of the D dropped limbs (last: what the
+// inverse low pass left), the lifts, and per remaining limb W's forward high
+// pass, stored for the low pass.  W need not be canonical there: fp64 limbs
+// take the centered lift of an fp64 prime as it is and 64-bit ones a word
+// below 4q, so a single dropped prime costs a target one addition.  The three
+// launches it replaced wrote and read W and the dropped limbs in coefficient
+// form: 12 polynomials of 13 limbs of 59 bits 48 us, now 26 us; two dropped
+// primes of a bootstrap's 16, the lift alone 136 us, now all three 137 us.  A block takes `per` targets; parts
+// repeat the dropped limbs' work (about one target's), so that few items fill
+// the chip.  grid (16, items, parts)
+template <int D>
+__global__ __launch_bounds__(TPB) void k_rescale_mid(Batch last, Batch w, int T, int per,
+                                                     const u64 *__restrict__ tab,
+                                                     const ModQ *__restrict__ mods, H4Tabs rt) {
+  const int cc = blockIdx.x * TPB + threadIdx.x;
+  const u64 *in = batch_ptr(last, blockIdx.y) + cc;
+  u64 *out = batch_ptr(w, blockIdx.y) + cc;
+  const u64 *tq = tab + 2 * (size_t)T, *tc = tq + 3 * (size_t)T * D;
+  u64 rv[D][16];
+#pragma unroll
+  for (int j = 0; j < D; j++) {
+    const int p = T + D - 1 - j;
+    const ModQ Mj = mods[p];
+    const u64 *ps = in + ((size_t)(D - 1 - j) << 16);
+    if (Mj.q < kFpPrimeBound) {
+      const double q = (double)Mj.q, qinv = 1.0 / q;
+      double x[16];
+#pragma unroll
+      for (int k = 0; k < 16; k++) x[k] = as_dbl(ps[4096 * k]);
+      fp_high_inv(x, rt.itw + ((size_t)p << 16), rt.ninv_fp[p], q, qinv);
+#pragma unroll
+      for (int k = 0; k < 16; k++) rv[j][k] = dbl_to_u52(x[k]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 16; k++) rv[j][k] = ps[4096 * k];
+      u64_high_inv(rv[j], rt.ipsi + ((size_t)p << 16), rt.ipsi_sh + ((size_t)p << 16),
+                   rt.ninv[2 * p], rt.ninv[2 * p + 1], lazy_q(Mj));
+    }
+#pragma unroll
+    for (int m = 0; m < j; m++) {
+      const u64 *cm = tc + 3 * ((size_t)j * D + m);
+      const u64 half = (mods[T + D - 1 - m].q - 1) / 2;
+#pragma unroll
+      for (int k = 0; k < 16; k++) {
+        u64 rm = barrett(0, rv[m][k], Mj);
+        if (rv[m][k] > half) rm = sub_mod(rm, cm[0], Mj.q);
+        rv[j][k] = shoup_mul(sub_mod(rv[j][k], rm, Mj.q), cm[1], cm[2], Mj.q);
+      }
+    }
+  }
+  const int i0 = blockIdx.z * per, i1 = min(i0 + per, T);
+  for (int i = i0; i < i1; i++) {
+    const ModQ M = mods[i];
+    const u64 *ti = tq + 3 * (size_t)i * D;
+    u64 *o = out + ((size_t)i << 16);
+    if (M.q < kFpPrimeBound) {
+      const double q = (double)M.q, qinv = 1.0 / q;
+      double x[16];
+#pragma unroll
+      for (int j = 0; j < D; j++) {
+        const u64 pj = mods[T + D - 1 - j].q;
+        const double wj = (double)ti[3 * j], wq = __dmul_rn(wj, qinv);
+#pragma unroll
+        for (int k = 0; k < 16; k++) {
+          // the centered lift, |v| < 2^44, or of a wide prime its residue
+          double v;
+          if (pj < kFpPrimeBound) {
+            v = u52_to_dbl(rv[j][k]);
+            if (rv[j][k] > (pj - 1) / 2) v = __dsub_rn(v, (double)pj);
+          } else {
+            u64 r = barrett(0, rv[j][k], M);
+            if (rv[j][k] > (pj - 1) / 2) r = sub_mod(r, ti[3 * j + 2], M.q);
+            v = u52_to_dbl(r);
+          }
+          x[k] = j ? __dadd_rn(x[k], fp_mulmod(v, wj, wq, q)) : v;
+        }
+      }
+      // |x| < 2^45 + 3q < 2^47 and at most q more a stage
+      fp_high_fwd(x, rt.tw + ((size_t)i << 16), q);
+#pragma unroll
+      for (int k = 0; k < 16; k++) o[4096 * k] = dbl_bits(x[k]);
+    } else {
+      const LazyQ Q = lazy_q(M);
+      u64 x[16];
+#pragma unroll
+      for (int j = 0; j < D; j++) {
+        const u64 pj = mods[T + D - 1 - j].q, neg = M.q - ti[3 * j + 2];
+        const bool small = pj <= 2 * M.q;
+#pragma unroll
+        for (int k = 0; k < 16; k++) {
+          // below 2q + q
+          const u64 r = (small ? rv[j][k] : barrett(0, rv[j][k], M)) +
+                        (rv[j][k] > (pj - 1) / 2 ? neg : 0);
+          // 3q + 4q before the reduction to below 3q
+          x[k] = j ? lazy_reduce(shoup_add(x[k], r, ti[3 * j], ti[3 * j + 1], Q), Q) : r;
+        }
+      }
+      u64_high_fwd(x, rt.psi + ((size_t)i << 16), rt.psi_sh + ((size_t)i << 16), Q);
+#pragma unroll
+      for (int k = 0; k < 16; k++) o[4096 * k] = x[k];
+    }
+  }
+}
+
+// (the columns of three dropped limbs leave one wave a SIMD, those of four go
+// to scratch memory)
+bool rescale_mid_ok(const ckks_context *c, int D) { return c->logN == 16 && D <= 2; }
+
+void launch_rescale_mid(ckks_context *c, const Batch &last, const Batch &w, int n_items, int limbs,
+                        int D, const u64 *tab) {
+  KTimer kt(c, "rescale", 8.0 * c->N * n_items * limbs,
+            (double)c->N * n_items * (limbs * D + 0.5 * 4 * limbs));
+  if (!rescale_mid_ok(c, D) || D < 1 || D >= limbs)
+    throw std::invalid_argument("rescale between the NTT halves: N = 2^16, 1 or 2 primes");
+  const int T = limbs - D;
+  // about four blocks a CU
+  const int parts = std::max(1, std::min(T, 4 * kCUs / (16 * n_items)));
+  const int per = (T + parts - 1) / parts;
+  hipLaunchKernelGGL(D == 1 ? k_rescale_mid<1> : k_rescale_mid<2>,
+                     dim3(16, n_items, (T + per - 1) / per), dim3(TPB), 0, c->stream, last, w, T, per,
+                     tab, c->d_mods, h4_tabs(c));
+  LAUNCH_CHECK();
+}
+
 // out_i = (src_i - w_i) inv_i for the T remaining limbs; grid (N / 256, T, items)
 __global__ void k_rescale_finish(Batch src, Batch w, Batch out, int logN,
                                  const u64 *__restrict__ inv, const ModQ *__restrict__ mods) {

@@ -831,6 +831,37 @@ def test_keyswitch_small_batches_full_size(params, levels):
 
 @pytest.mark.slow
 @pytest.mark.parametrize("params", [
+    dict(log_n=16, depth=9, dnum=2, dcrt_bits=40, first_mod=60, special_bits=60),
+    # primes of 2^45 or more, dropped from above limbs of the same size
+    dict(log_n=16, depth=9, dnum=2, dcrt_bits=59, first_mod=60, special_bits=60),
+    # primes on both sides of the 2^45 bound of the fp64 path
+    dict(log_n=16, depth=9, dnum=2, dcrt_bits=45, first_mod=60, special_bits=60),
+    # a wide first prime above narrower limbs
+    dict(log_n=16, depth=9, dnum=2, dcrt_bits=50, first_mod=60, special_bits=60),
+], ids=["40", "59", "45", "50"])
+def test_rescale_full_size(params):
+    """Rescales by 1 to 3 primes at N = 2^16, at the levels where every limb, a
+    few and one are left, of one ciphertext and of batches: the oracle's words."""
+    fhe = _fhe()
+    client, ctx, orc = _pair(params)
+    rng = np.random.default_rng(5)
+    zs = [rng.uniform(-1, 1, 64) for _ in range(3)]
+    for limbs in (10, 5, 2):
+        cts = [client.encrypt(z, slots=64, cur_limbs=limbs, enc_id=800 + i)
+               for i, z in enumerate(zs)]
+        want = [orc.encrypt(z, slots=64, scale=ctx.scale_at(limbs), limbs=limbs, enc_id=800 + i)
+                for i, z in enumerate(zs)]
+        for k in range(1, min(3, limbs - 1) + 1):
+            want = [orc.rescale(w) for w in want]
+            for batch in (cts[:1], cts, cts * 9):
+                got = fhe.rescale_many(batch, ctx, primes=k)
+                for i, g in enumerate(got):
+                    assert np.array_equal(g.download(), want[i % 3]), (limbs, k, len(batch), i)
+    ctx.close()
+
+
+@pytest.mark.slow
+@pytest.mark.parametrize("params", [
     "keyswitch",
     dict(log_n=16, depth=9, dnum=2, dcrt_bits=59, first_mod=60, special_bits=60),
     dict(log_n=15, depth=5, dnum=3, dcrt_bits=40, first_mod=60, special_bits=60),
