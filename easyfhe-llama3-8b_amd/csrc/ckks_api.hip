@@ -1117,8 +1117,12 @@ static bool ks_modup(ckks_context *c, int limbs, int n, const u64 *const *d, u64
 }
 
 // A batched key switch is split into parts of at least this many items
-// (run_parts)
-constexpr int kSplitMin = 8;
+// (run_parts).  On 64-bit special primes parts of 3 pay: 6 to 12 ciphertexts
+// of 26 limbs 3 to 7% (6: 914 -> 855 us a rotation, 1130 -> 1028 a product),
+// of 8 limbs 4 to 8%.  On fp64 ones, whose kernels are shorter, the gain at 6
+// (3 to 9%) is lost again at 8 of 12 limbs (377 -> 396 us): 8, as measured
+// with whole batches.
+static int split_min(const ckks_context *c) { return low_key_special_fp(c) ? 8 : 3; }
 
 struct KsJob {
   int ext_item;
@@ -1327,7 +1331,7 @@ static u64 galois_inverse(const ckks_context *c, u64 g) {
 // blocks, 48 more than run at once, and 84 us against 65 us with 3 limbs
 // moved (the other two launches 3 us longer).
 static int defer_from(const ckks_context *c, int n, int limbs) {
-  if (n >= 2 * kSplitMin) return 0;  // parts on other streams fill the gaps
+  if (n >= 16) return 0;  // several rounds: their overlap hides a short last one
   const int slots = 2 * kCUs, per = 16 * n;
   int fp = 0, other = c->alpha;
   for (int l = 0; l < limbs; l++) (c->prime_fp[l] ? fp : other)++;
@@ -1440,7 +1444,7 @@ static void gen_key(ckks_context *c, u64 id, int relin, u64 galois) {
 // which waits for everything issued before it (its inputs) and is joined
 // back before the function returns; every part's intermediates stay
 // allocated until then, so that no block of one part is handed to another
-// while still in use.  Parts keep at least kSplitMin items.
+// while still in use.  Parts keep at least split_min items.
 struct StreamSwap {
   ckks_context *c;
   hipStream_t saved;
@@ -1450,7 +1454,7 @@ struct StreamSwap {
 
 template <typename F>
 static void run_parts(ckks_context *c, int b0, int nb, F run) {
-  const int parts = std::min(c->split_parts, std::max(1, nb / kSplitMin));
+  const int parts = std::min(c->split_parts, std::max(1, nb / split_min(c)));
   if (parts <= 1) {
     Scratch s(c);
     run(b0, nb, s);
