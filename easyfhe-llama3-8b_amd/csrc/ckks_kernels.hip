@@ -1,6 +1,7 @@
 // ckks_kernels.hip -- gfx950 kernels of the RNS-CKKS backend.
 //
-// All kernels use 256-thread workgroups (four wave64s).  Polynomials are
+// Kernels use 256-thread workgroups (four wave64s), but for the whole-ring ones
+// (up to 1024 threads).  Polynomials are
 // uint64 limb arrays of N residues; the NTT domain is the bit-reversed
 // evaluation order a_hat[i] = a(psi^(2 br(i) + 1)).
 #include <math.h>
@@ -30,7 +31,8 @@ namespace ckks {
 constexpr int TPB = 256;
 
 // ===========================================================================
-// NTT: two passes of LDS-staged radix-2 stages.
+// NTT of N = 2^15 and 2^17: two passes of LDS-staged radix-2 stages (2^10 ..
+// 2^14: the whole-ring kernels; 2^16: the register passes).
 //   high pass: bit positions [logN - S1, logN), a tile is 2^S1 rows (stride
 //              N / 2^S1) by C adjacent columns, so global loads stay
 //              coalesced in C-element runs;
