@@ -3333,7 +3333,11 @@ struct H4Job {
 struct H4Jobs {
   H4Job j[kMaxDigits];
 };
-template <int NK, int RSD = 0>
+// WIDE_DROP: a dropped prime is 2^45 or more.  An instance of its own: with the
+// choice between the two kinds of dropped word in every row, the 40-bit chain's
+// form took 2 to 17% longer (96 polynomials of 36 + 12 limbs, one dropped prime,
+// 1063 us against 990; of 6 + 12 limbs, two dropped primes, 711 against 607).
+template <int NK, int RSD = 0, bool WIDE_DROP = false>
 __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
     Batch src, Batch dst, H4Jobs jobs, int split, int q_limbs, int L,
     const ModQ *__restrict__ mods, H4Tabs nt, const u64 *__restrict__ rs,
@@ -3611,7 +3615,8 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
               // a mask select, so that y keeps static indices
               const u64 msk = 0ull - (u64)ee_d;
               const u64 yr = (y[0][r] & ~msk) | (y[1][r] & msk);
-              const u64 yd = qd < kFpPrimeBound ? fp_canon(as_dbl(yr), qinv, q) : yr;
+              const u64 yd =
+                  WIDE_DROP && qd >= kFpPrimeBound ? yr : fp_canon(as_dbl(yr), qinv, q);
               u64 u = shoup_mul(sub_mod(xs[4096 * r], yd, qd), pinv, pinvs, qd);
 #pragma unroll
               for (int m = 0; m < j; m++) {
@@ -3650,7 +3655,8 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
             }
           } else {
             // y + r_j f (- f p) with f = [P p_1..p_j]_t by its Shoup constant,
-            // lazily: below 2q + 4q with the correction, reduced to below 3q
+            // lazily: y (below q, after the first lift below 3q), the
+            // correction and the product below 8q, reduced to below 3q
             const u64 qu = w[0], f = w[10 + 4 * j], fs = w[11 + 4 * j], neg = qu - w[13 + 4 * j];
             const LazyQ Q{qu, 0 - qu, (u32)ttw[(size_t)t * 32 + 16], 0, 0};
 #pragma unroll
@@ -3914,14 +3920,25 @@ void launch_convert_h4_rs(ckks_context *c, const Batch &src, const Batch &dst, i
   const int T = t.nd - D;
   const double2 *rsf =
       (const double2 *)(rtab + 2 * (size_t)T * D + 2 * (size_t)D + 3 * (size_t)D * D);
-  auto k1 = t.n_k == 1 ? k_convert_h4<1, 1> : t.n_k == 2 ? k_convert_h4<2, 1> : k_convert_h4<3, 1>;
-  auto k2 = t.n_k == 1 ? k_convert_h4<1, 2> : t.n_k == 2 ? k_convert_h4<2, 2> : k_convert_h4<3, 2>;
+  bool wide_drop = false;
+  for (int j = 0; j < D; j++) wide_drop = wide_drop || !c->prime_fp[t.nd - 1 - j];
+  auto pick = [&](auto d, auto w) {
+    constexpr int RSD = decltype(d)::value;
+    constexpr bool WD = decltype(w)::value;
+    return t.n_k == 1   ? k_convert_h4<1, RSD, WD>
+           : t.n_k == 2 ? k_convert_h4<2, RSD, WD>
+                        : k_convert_h4<3, RSD, WD>;
+  };
+  const std::integral_constant<int, 1> d1;
+  const std::integral_constant<int, 2> d2;
+  auto kern = wide_drop ? (D == 1 ? pick(d1, std::true_type{}) : pick(d2, std::true_type{}))
+                        : (D == 1 ? pick(d1, std::false_type{}) : pick(d2, std::false_type{}));
   const int flags = 1 | h4_wide_sources(c, src, n_items, t.ns, c->L, t.nd) |
                     h4_wide_targets(c, dst, n_items, T, t.nd, 0, t.nd, false);
   H4Jobs jobs{};
   jobs.j[0] = H4Job{t.sn, t.mt, 0, 0, t.ns, t.nd, t.n_tg, t.wide_mask, c->L, t.nd, 0, flags};
   const int passes = (t.nd + 7) >> 3, split = h4_split(64 * n_items, std::max(1, passes - 1));
-  hipLaunchKernelGGL(D == 1 ? k1 : k2, dim3(64, n_items, split), dim3(TPB), convert_h4_lds(t, D),
+  hipLaunchKernelGGL(kern, dim3(64, n_items, split), dim3(TPB), convert_h4_lds(t, D),
                      c->stream, src, dst, jobs, split, t.nd, c->L, c->d_mods, h4_tabs(c), rtab, rsf);
   LAUNCH_CHECK();
   if (flags & 4) h4_wide_targets(c, dst, n_items, T, t.nd, 0, t.nd, true);

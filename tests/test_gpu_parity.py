@@ -830,6 +830,39 @@ def test_keyswitch_small_batches_full_size(params, levels):
 
 
 @pytest.mark.slow
+@pytest.mark.parametrize("params,levels", [
+    # both dropped targets in one pass of 8 beside two (19), one (10) and no
+    # (5) further passes, and in two passes (17 and 9: the separate conversion)
+    (dict(log_n=16, depth=18, dnum=3, dcrt_bits=59, first_mod=60, special_bits=60),
+     (19, 17, 10, 9, 5)),
+    # primes on both sides of the fp64 path's bound of 2^45
+    (dict(log_n=16, depth=9, dnum=2, dcrt_bits=45, first_mod=60, special_bits=60), (10, 5)),
+], ids=["59", "45"])
+def test_two_prime_products_on_wide_chains_full_size(params, levels):
+    """Relinearise-rescales by two primes of 2^45 or more at N = 2^16: the
+    oracle's words, for one ciphertext and batches (split and whole
+    conversions)."""
+    fhe = _fhe()
+    client, ctx, orc = _pair(params)
+    rng = np.random.default_rng(13)
+    zs = [rng.uniform(-1, 1, 64) for _ in range(3)]
+    for limbs in levels:
+        cts = [client.encrypt(z, slots=64, cur_limbs=limbs, enc_id=450 + i)
+               for i, z in enumerate(zs)]
+        refs = [orc.encrypt(z, slots=64, scale=ctx.scale_at(limbs), limbs=limbs, enc_id=450 + i)
+                for i, z in enumerate(zs)]
+        want = [orc.rescale(orc.rescale(orc.relinearize(orc.tensor(refs[i], refs[i - 1]))))
+                for i in range(3)]
+        for n in (1, 2, 3, 9):
+            left = [cts[i % 3] for i in range(n)]
+            right = [cts[(i - 1) % 3] for i in range(n)]
+            got = fhe.homo_mul_relin_rescale_many(left, right, ctx, primes=2)
+            for i in range(n):
+                assert np.array_equal(got[i].download(), want[i % 3]), (limbs, n, i)
+    ctx.close()
+
+
+@pytest.mark.slow
 @pytest.mark.parametrize("params", [
     dict(log_n=16, depth=9, dnum=2, dcrt_bits=40, first_mod=60, special_bits=60),
     # primes of 2^45 or more, dropped from above limbs of the same size
@@ -991,16 +1024,18 @@ def test_scalar_constants_and_invalid_objects():
 # a chain whose special primes are too wide for the merged relinearise-rescale
 # ModDown (12 x 60-bit P: the postop then runs as separate launches)
 WIDE_P = dict(log_n=12, depth=35, dnum=3, dcrt_bits=40, first_mod=60, special_bits=60)
+# N = 2^16 with dropped and kept primes of 2^45 or more only
+WIDE_Q = dict(log_n=16, depth=9, dnum=2, dcrt_bits=59, first_mod=60, special_bits=60)
 
 
-@pytest.mark.parametrize("name", ["small", "matvec", "keyswitch", "wide_p"])
+@pytest.mark.parametrize("name", ["small", "matvec", "keyswitch", "wide_p", "wide_q"])
 def test_mul_relin_rescale_postop_matches_composed(name):
     """homo_mul_relin_rescale_postop (x2, - sub, + scalar folded into the
     ModDown epilogue) equals the oracle's relinearise, rescale, add, sub and
     scalar add on the same words (reference operators/nonlinear/
     polynomial.py:115-203: 2 T_i T_j - T_1 and 2 T_i T_j - 1)."""
     fhe = _fhe()
-    p = WIDE_P if name == "wide_p" else name
+    p = {"wide_p": WIDE_P, "wide_q": WIDE_Q}.get(name, name)
     client, ctx = device_context(p)
     orc = oracle_context(p)
     orc.gen_relin_key()
