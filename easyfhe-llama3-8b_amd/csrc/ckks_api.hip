@@ -1116,13 +1116,25 @@ static bool ks_modup(ckks_context *c, int limbs, int n, const u64 *const *d, u64
   return false;
 }
 
-// A batched key switch is split into parts of at least this many items
-// (run_parts).  On 64-bit special primes parts of 3 pay: 6 to 12 ciphertexts
-// of 26 limbs 3 to 7% (6: 914 -> 855 us a rotation, 1130 -> 1028 a product),
-// of 8 limbs 4 to 8%.  On fp64 ones, whose kernels are shorter, the gain at 6
-// (3 to 9%) is lost again at 8 of 12 limbs (377 -> 396 us): 8, as measured
-// with whole batches.
-static int split_min(const ckks_context *c) { return low_key_special_fp(c) ? 8 : 3; }
+// Parts of a batched key switch of n ciphertexts at `limbs` limbs (run_parts):
+// of at least 8 items.  On 64-bit special primes (fp64 kernels are shorter)
+// and N >= 2^15 parts of 3 pay too where the work covers the launches that
+// every part repeats: p parts from p^2 2^18 words of a polynomial on.  One
+// part against two (us a rotation): N = 2^16, 6 x 26 limbs 922 / 856, 7 x 4
+// limbs 233 / 219, 6 x 2 limbs 165 / 167 (a product 213 / 221), 7 x 2 limbs of
+// a 40-bit chain 169 / 172 (213 / 227); N = 2^15, 9 x 4 limbs 466 / 454, 8 x 4
+// 435 / 438, 12 x 2 270 / 275.  Two against three: N = 2^15, 16 x 4 limbs 518 /
+// 541, 16 x 10 630 / 623.  The whole-ring kernels are shorter yet: N = 2^12, 9 x
+// 4 limbs 52 / 80 / 116 in one, two and three.  On fp64 special primes parts of
+// 3 gain 3 to 9% at 6 ciphertexts and lose 5% at 8 of 12 limbs: 8.
+static int split_count(const ckks_context *c, int n, int limbs) {
+  int parts = std::max(1, n / 8);
+  if (c->logN >= 15 && !low_key_special_fp(c)) {
+    const u64 words = ((u64)n * limbs) << c->logN;
+    while (3 * (parts + 1) <= n && words > (u64)(parts + 1) * (parts + 1) << 18) parts++;
+  }
+  return std::min(c->split_parts, parts);
+}
 
 struct KsJob {
   int ext_item;
@@ -1444,7 +1456,7 @@ static void gen_key(ckks_context *c, u64 id, int relin, u64 galois) {
 // which waits for everything issued before it (its inputs) and is joined
 // back before the function returns; every part's intermediates stay
 // allocated until then, so that no block of one part is handed to another
-// while still in use.  Parts keep at least split_min items.
+// while still in use.
 struct StreamSwap {
   ckks_context *c;
   hipStream_t saved;
@@ -1453,8 +1465,8 @@ struct StreamSwap {
 };
 
 template <typename F>
-static void run_parts(ckks_context *c, int b0, int nb, F run) {
-  const int parts = std::min(c->split_parts, std::max(1, nb / split_min(c)));
+static void run_parts(ckks_context *c, int b0, int nb, int limbs, F run) {
+  const int parts = split_count(c, nb, limbs);
   if (parts <= 1) {
     Scratch s(c);
     run(b0, nb, s);
@@ -1523,7 +1535,7 @@ static void rotate_batch(ckks_context *c, const ckks_ct *const *in, int n, u64 g
       run(b0, nb, s);
       if (arena_used) *arena_used = std::max(*arena_used, s.used);
     } else {
-      run_parts(c, b0, nb, run);
+      run_parts(c, b0, nb, limbs, run);
     }
   }
 }
@@ -1547,7 +1559,8 @@ static void relin_batch(ckks_context *c, const ckks_ct *const *in, int n, ckks_c
     u64 *acc = ks_modup_inner(c, limbs, nb, d.data(), jobs, s, &sp, &sp_done, &dk);
     ks_moddown(c, limbs, acc, jobs, s, ptmp, sp_done, &dk);
   };
-  for (int b0 = 0; b0 < n; b0 += kMaxBatch) run_parts(c, b0, std::min(kMaxBatch, n - b0), run);
+  for (int b0 = 0; b0 < n; b0 += kMaxBatch)
+    run_parts(c, b0, std::min(kMaxBatch, n - b0), limbs, run);
 }
 
 // Relinearisation of n degree-2 ciphertexts followed by D rescales, as one
@@ -1696,7 +1709,8 @@ static void relin_rescale_batch(ckks_context *c, const ckks_ct *const *in, int n
                              gal.data(), o0, o1, nb, T, E, rt, amul, &po);
     }
   };
-  for (int b0 = 0; b0 < n; b0 += kMaxBatch) run_parts(c, b0, std::min(kMaxBatch, n - b0), run);
+  for (int b0 = 0; b0 < n; b0 += kMaxBatch)
+    run_parts(c, b0, std::min(kMaxBatch, n - b0), limbs, run);
 }
 
 // Constants of a rescale by the last D primes p_1 = q_{limbs-1}, p_2, ... of

@@ -396,7 +396,7 @@ struct ckks_context {
   // special limbs' conversion; environment CKKS_KS_DEFER=0 at creation keeps
   // the accumulators in HBM between the two
   bool ks_defer = true;
-  // batched key switches of at least split_min ciphertexts per part run as
+  // batched key switches of at least 3 ciphertexts per part (split_count) run as
   // `split_parts` parts, the first on the context stream and the others on
   // `aux` streams (forked from and joined back into the context stream), so
   // that a latency-bound kernel of one part shares the CUs with a streaming

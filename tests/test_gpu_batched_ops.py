@@ -35,3 +35,43 @@ def test_add_many_matches_pairwise_adds():
     for c in a + b + [low]:
         c.release()
     ctx.close()
+
+
+@pytest.mark.parametrize("params,expected", [
+    # whole-ring kernels: parts of 8
+    (dict(log_n=10, depth=9, dnum=2, dcrt_bits=40, first_mod=60, special_bits=60),
+     {(5, 9): 1, (10, 12): 1, (10, 16): 2}),
+    # 64-bit special primes from N = 2^15 on: by the words of the batch
+    (dict(log_n=15, depth=3, dnum=4, dcrt_bits=40, first_mod=40, special_bits=60),
+     {(2, 12): 1, (4, 8): 1, (4, 9): 2, (4, 16): 2, (2, 16): 2}),
+    (dict(log_n=16, depth=9, dnum=2, dcrt_bits=59, first_mod=60, special_bits=60),
+     {(2, 6): 1, (10, 5): 1, (10, 6): 2, (10, 9): 3}),
+    # fp64 special primes: parts of 8
+    (dict(log_n=16, depth=3, dnum=2, dcrt_bits=40, first_mod=40, special_bits=44),
+     {(4, 12): 1, (4, 16): 2}),
+], ids=["ring", "2^15", "wide", "fp64"])
+def test_batched_rotations_run_in_as_many_parts_as_pay(params, expected):
+    """A batched key switch repeats its launches in every part, so short
+    batches stay whole (one key product a part); the words are the single
+    rotations' however it is split."""
+    from easyfhe import fhe
+
+    client, ctx = device_context(params, rotations=(3,))
+    rng = np.random.default_rng(8)
+    for (limbs, n), parts in expected.items():
+        cts = [client.encrypt(rng.uniform(-1, 1, 16), slots=16, cur_limbs=limbs, enc_id=i)
+               for i in range(n)]
+        want = [fhe.homo_rotate(c, 3, ctx).download() for c in cts]
+        for split, runs in ((0, parts), (1, 1)):
+            ctx.set_split_parts(split)
+            ctx.profile(True)
+            ctx.profile_read()
+            got = fhe.homo_rotate_many(cts, 3, ctx)
+            launched = ctx.profile_read()
+            ctx.profile(False)
+            assert sum(launched[k]["launches"] for k in ("key_inner", "ntt_low_key")
+                       if k in launched) == runs, (limbs, n, split)
+            for g, w in zip(got, want):
+                assert np.array_equal(g.download(), w), (limbs, n, split)
+        ctx.set_split_parts(0)
+    ctx.close()
