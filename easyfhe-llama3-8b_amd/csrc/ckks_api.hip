@@ -1151,6 +1151,7 @@ struct KsDeferred {
   // input: the Q limbs [0, below) whose key product may be deferred (-1: all,
   // where ks_moddown's tile conversion applies)
   int below = -1;
+  bool alone = false;  // input: no other part runs beside this one
   bool on = false;
   int from = 0;  // the limbs deferred: fp64 ones from here on
   const u64 *ext = nullptr;
@@ -1341,7 +1342,10 @@ static u64 galois_inverse(const ckks_context *c, u64 g) {
 // All of them, unless a last round of few blocks can move whole into the free
 // slots of the special limbs' launch: one ciphertext of 35 fp64 limbs is 560
 // blocks, 48 more than run at once, and 84 us against 65 us with 3 limbs
-// moved (the other two launches 3 us longer).
+// moved (the other two launches 3 us longer).  For a batch on one stream only
+// (KsDeferred::alone): where parts run beside one another a short last round
+// is filled by the others, and the moved limbs' accumulators are read and
+// written for nothing (24 rotations of 12 limbs 929 us with, 902 without).
 static int defer_from(const ckks_context *c, int n, int limbs) {
   if (n >= 16) return 0;  // several rounds: their overlap hides a short last one
   const int slots = 2 * kCUs, per = 16 * n;
@@ -1393,7 +1397,7 @@ static u64 *ks_modup_inner(ckks_context *c, int limbs, int n, const u64 *const *
   if (dk) {
     dk->on = defer;
     if (defer) {
-      dk->from = dk->below >= 0 ? 0 : defer_from(c, n, limbs);
+      dk->from = dk->below >= 0 || !dk->alone ? 0 : defer_from(c, n, limbs);
       dk->ext = ext;
       dk->est = est;
       dk->own = ob;
@@ -1469,7 +1473,7 @@ static void run_parts(ckks_context *c, int b0, int nb, int limbs, F run) {
   const int parts = split_count(c, nb, limbs);
   if (parts <= 1) {
     Scratch s(c);
-    run(b0, nb, s);
+    run(b0, nb, s, true);
     return;
   }
   std::vector<std::unique_ptr<Scratch>> sc;
@@ -1479,10 +1483,10 @@ static void run_parts(ckks_context *c, int b0, int nb, int limbs, F run) {
   for (int i = 0; i < parts; i++) {
     const int lo = b0 + nb * i / parts, hi = b0 + nb * (i + 1) / parts;
     if (i == 0) {
-      run(lo, hi - lo, *sc[i]);
+      run(lo, hi - lo, *sc[i], false);
     } else {
       StreamSwap sw(c, c->aux[i - 1]);
-      run(lo, hi - lo, *sc[i]);
+      run(lo, hi - lo, *sc[i], false);
     }
   }
   for (int i = 1; i < parts; i++) {
@@ -1513,7 +1517,7 @@ static void rotate_batch(ckks_context *c, const ckks_ct *const *in, int n, u64 g
   const int limbs = in[0]->limbs;
   const size_t N = c->N, P = (size_t)limbs * N;
   const DeviceKey &key = get_key(c, g);
-  auto run = [&](int b0, int nb, Scratch &s) {
+  auto run = [&](int b0, int nb, Scratch &s, bool alone) {
     std::vector<const u64 *> d(nb);
     for (int i = 0; i < nb; i++) d[i] = in[b0 + i]->d + P;
     std::vector<KsJob> jobs(nb);
@@ -1524,6 +1528,7 @@ static void rotate_batch(ckks_context *c, const ckks_ct *const *in, int n, u64 g
     const Strided sp{ptmp, (u64)c->alpha * N};
     bool sp_done = false;
     KsDeferred dk;
+    dk.alone = alone;
     u64 *acc = ks_modup_inner(c, limbs, nb, d.data(), jobs, s, &sp, &sp_done, &dk);
     ks_moddown(c, limbs, acc, jobs, s, ptmp, sp_done, &dk);
   };
@@ -1532,7 +1537,7 @@ static void rotate_batch(ckks_context *c, const ckks_ct *const *in, int n, u64 g
     if (arena) {
       // the fixed scratch holds one batch's intermediates: one stream
       Scratch s(c, arena, arena_words);
-      run(b0, nb, s);
+      run(b0, nb, s, true);
       if (arena_used) *arena_used = std::max(*arena_used, s.used);
     } else {
       run_parts(c, b0, nb, limbs, run);
@@ -1545,7 +1550,7 @@ static void relin_batch(ckks_context *c, const ckks_ct *const *in, int n, ckks_c
   const int limbs = in[0]->limbs;
   const size_t N = c->N, P = (size_t)limbs * N;
   const DeviceKey &key = get_key(c, 0);
-  auto run = [&](int b0, int nb, Scratch &s) {
+  auto run = [&](int b0, int nb, Scratch &s, bool alone) {
     std::vector<const u64 *> d(nb);
     for (int i = 0; i < nb; i++) d[i] = in[b0 + i]->d + 2 * P;
     std::vector<KsJob> jobs(nb);
@@ -1556,6 +1561,7 @@ static void relin_batch(ckks_context *c, const ckks_ct *const *in, int n, ckks_c
     const Strided sp{ptmp, (u64)c->alpha * N};
     bool sp_done = false;
     KsDeferred dk;
+    dk.alone = alone;
     u64 *acc = ks_modup_inner(c, limbs, nb, d.data(), jobs, s, &sp, &sp_done, &dk);
     ks_moddown(c, limbs, acc, jobs, s, ptmp, sp_done, &dk);
   };
@@ -1601,7 +1607,7 @@ static void relin_rescale_batch(ckks_context *c, const ckks_ct *const *in, int n
   const DeviceKey &key = get_key(c, 0);
   const BCTable &bt = bc_down(c, limbs);
   const u64 *rt = relin_rs_table(c, limbs, D);
-  auto run = [&](int b0, int nb, Scratch &s) {
+  auto run = [&](int b0, int nb, Scratch &s, bool) {
     Batch fa{}, fb{}, fb1{};
     const Batch prod = strided(in[b0]->d, 3 * P);
     std::vector<const u64 *> d(nb);

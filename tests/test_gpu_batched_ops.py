@@ -75,3 +75,27 @@ def test_batched_rotations_run_in_as_many_parts_as_pay(params, expected):
                 assert np.array_equal(g.download(), w), (limbs, n, split)
         ctx.set_split_parts(0)
     ctx.close()
+
+
+def test_split_batches_keep_the_fused_combine():
+    """Limbs move out of the fused key product + combine only where a batch
+    runs alone: of 24 rotations at 12 limbs (three parts) the separate combine
+    takes q_0 alone, of one at 36 limbs a last round's limbs too."""
+    from easyfhe import fhe
+
+    client, ctx = device_context("keyswitch", rotations=(3,), relin=False)
+    rng = np.random.default_rng(9)
+    for limbs, n, runs in ((12, 24, 1), (36, 1, 4)):
+        cts = [client.encrypt(rng.uniform(-1, 1, 16), slots=16, cur_limbs=limbs, enc_id=i)
+               for i in range(n)]
+        want = [fhe.homo_rotate(c, 3, ctx).download() for c in cts]
+        ctx.profile(True)
+        ctx.profile_read()
+        got = fhe.homo_rotate_many(cts, 3, ctx)
+        # accumulators, converted words and outputs of two components, one addend
+        words = ctx.profile_read()["ntt_fwd_moddown"]["bytes"] / (8.0 * (1 << 16) * 7 * n)
+        ctx.profile(False)
+        assert round(words, 3) == runs, (limbs, n)
+        for g, w in zip(got, want):
+            assert np.array_equal(g.download(), w), (limbs, n)
+    ctx.close()
