@@ -1479,6 +1479,18 @@ static void run_parts(ckks_context *c, int b0, int nb, int limbs, F run) {
   std::vector<std::unique_ptr<Scratch>> sc;
   for (int i = 0; i < parts; i++) sc.emplace_back(new Scratch(c));
   HIPCHECK(hipEventRecord(c->fork_ev, c->stream));
+  // the context stream waits for the others also where a part throws, before
+  // the parts' intermediates go back to the pool
+  struct Join {
+    ckks_context *c;
+    int n;
+    ~Join() {
+      for (int i = 0; i < n; i++) {
+        (void)hipEventRecord(c->join_ev[i], c->aux[i]);
+        (void)hipStreamWaitEvent(c->stream, c->join_ev[i], 0);
+      }
+    }
+  } join{c, parts - 1};
   for (int i = 1; i < parts; i++) HIPCHECK(hipStreamWaitEvent(c->aux[i - 1], c->fork_ev, 0));
   for (int i = 0; i < parts; i++) {
     const int lo = b0 + nb * i / parts, hi = b0 + nb * (i + 1) / parts;
@@ -1493,6 +1505,7 @@ static void run_parts(ckks_context *c, int b0, int nb, int limbs, F run) {
     HIPCHECK(hipEventRecord(c->join_ev[i - 1], c->aux[i - 1]));
     HIPCHECK(hipStreamWaitEvent(c->stream, c->join_ev[i - 1], 0));
   }
+  join.n = 0;
 }
 
 // Words of key-switch scratch that rotate_batch takes for nb ciphertexts at
