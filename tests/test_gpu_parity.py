@@ -111,9 +111,8 @@ def test_encrypt_decrypt_parity(name):
 
 @pytest.mark.parametrize("slots", [2, 64, 2048])
 def test_encrypt_input_forms(slots):
-    """Real, complex, integer and short inputs, and a buffer overwritten right
-    after the call, give the oracle's limbs; rows below, at and above the
-    register FFT's tile."""
+    """Real, complex, integer and short inputs give the oracle's limbs; rows
+    below and at the register FFT's tile."""
     fhe = _fhe()
     client, ctx = device_context("small", relin=False)
     orc = oracle_context("small")
@@ -126,12 +125,42 @@ def test_encrypt_input_forms(slots):
         pad = np.zeros(slots, dtype=np.complex128)
         pad[: len(z)] = z
         want = orc.encrypt(pad, slots=slots, scale=sc, limbs=ctx.L, enc_id=60 + i)
-        buf = np.array(z)
-        ct = client.encrypt(buf, slots=slots, enc_id=60 + i)
-        buf[:] = 7
+        ct = client.encrypt(z, slots=slots, enc_id=60 + i)
         assert np.array_equal(ct.download(), want), i
         # noise of a fresh encryption at scale 2^40
         assert np.abs(client.decrypt_complex(ct) - pad).max() < 1e-6
+
+
+def test_encrypt_leaves_the_callers_buffers_free():
+    """The native call copies its inputs before it returns: arrays overwritten
+    right after it, and used again for the next call, give the oracle's limbs
+    in every one of several calls in a row."""
+    import ctypes
+
+    from easyfhe import _native
+
+    fhe = _fhe()
+    client, ctx = device_context("small", relin=False)
+    orc = oracle_context("small")
+    rng = np.random.default_rng(77)
+    slots, sc = 2048, ctx.scale_at(ctx.L)
+    re, im = np.empty(slots), np.empty(slots)
+    zs = rng.uniform(-1, 1, (24, slots)) + 1j * rng.uniform(-1, 1, (24, slots))
+    cts = []
+    for i, z in enumerate(zs):
+        re[:], im[:] = z.real, z.imag
+        out = ctypes.c_void_p()
+        real_only = i % 3 == 2
+        _native.check(_native.lib.ckks_encrypt(
+            ctx.handle, re.ctypes.data_as(_native.DP),
+            None if real_only else im.ctypes.data_as(_native.DP), slots, ctx.L, sc, 900 + i,
+            ctypes.byref(out)))
+        re[:] = im[:] = 7.0
+        cts.append(fhe._wrap(ctx, out))
+    for i, (z, ct) in enumerate(zip(zs, cts)):
+        z = z.real.astype(complex) if i % 3 == 2 else z
+        want = orc.encrypt(z, slots=slots, scale=sc, limbs=ctx.L, enc_id=900 + i)
+        assert np.array_equal(ct.download(), want), i
 
 
 def test_encode_parity_large_scale():
@@ -1109,15 +1138,18 @@ def test_align_to_changes_the_scale():
         fhe.align_to(ct, ct.state.replace(scaling_factor=ct.state.scaling_factor * 1.5), ctx)
 
 
-@pytest.mark.parametrize("first_mod,dcrt_bits,special_bits", [(46, 46, 47), (53, 50, 59), (60, 59, 60)])
+@pytest.mark.parametrize("log_n", [10, 11, 12, 13, 14, 16])
+@pytest.mark.parametrize("first_mod,dcrt_bits,special_bits",
+                         [(43, 43, 44), (46, 46, 47), (53, 50, 59), (60, 59, 60)])
 @pytest.mark.parametrize("fill", ["max", "alternate", "one_max"])
-def test_ntt_lazy_bounds_full_size(fill, first_mod, dcrt_bits, special_bits):
-    """The 64-bit transforms at N = 2^16 over their range of primes (46 to 60
-    bits), on words that drive the unreduced sums to their ends: every word
+def test_ntt_lazy_bounds(fill, first_mod, dcrt_bits, special_bits, log_n):
+    """The 64-bit transforms of the whole-ring kernels and of N = 2^16 over
+    their range of primes (46 to 60 bits), and the fp64 ones at their largest
+    primes, on words that drive the unreduced sums to their ends: every word
     q - 1, q - 1 and 0 in turn, one non-zero word."""
     from easyfhe import _native
 
-    p = dict(log_n=16, depth=3, dnum=2, dcrt_bits=dcrt_bits, first_mod=first_mod,
+    p = dict(log_n=log_n, depth=3, dnum=2, dcrt_bits=dcrt_bits, first_mod=first_mod,
              special_bits=special_bits)
     client, ctx = device_context(p, relin=False)
     orc = oracle_context(p)
@@ -1130,7 +1162,7 @@ def test_ntt_lazy_bounds_full_size(fill, first_mod, dcrt_bits, special_bits):
         elif fill == "alternate":
             a[0, l, ::2] = top
         else:
-            a[0, l, 4097 * (l + 1)] = top
+            a[0, l, 4097 * (l + 1) % N] = top
     for inverse, exp in ((0, orc.ntt_limbs(a[0], q_limbs=L)), (1, orc.intt_limbs(a[0], q_limbs=L))):
         got = np.zeros_like(a)
         _native.check(_native.lib.ckks_poly_ntt(ctx.handle, a.ctypes.data_as(_native.U64P),
