@@ -643,7 +643,8 @@ __device__ __forceinline__ void k_ntt16_fwd_low_body(u64 *__restrict__ lds, Batc
   }
 }
 
-// inverse, bit positions 0..11 (first pass): input in [0, 2q), output in [0, 8q]
+// inverse, bit positions 0..11 (first pass): input in [0, 3q) (a product formed
+// on load), output in [0, 8q]
 __device__ __forceinline__ void k_ntt16_inv_low_body(u64 *__restrict__ lds, Batch src, Batch dst, int l_begin,
                                                        int q_limbs, int L,
                                                        const ModQ *__restrict__ mods,
@@ -1215,7 +1216,8 @@ struct Ring {
 };
 
 // the next round's twiddles before a round's butterflies (8 words a thread) or
-// after them (16 words: two sets of 15 do not fit 128 registers)
+// after them (16 words: a block of 1024 threads leaves a thread 128 registers,
+// and with one set of 15 pairs the N = 2^14 kernels already spill 40 to 72)
 template <int LW>
 constexpr bool kEarly = LW <= 3;
 
@@ -1619,8 +1621,11 @@ __global__ __launch_bounds__((1 << (LOGN - LW))) void k_ring_moddown(RingModDown
   u64 *o = (comp ? io.out1 : io.out0) + ((size_t)l << LOGN) + t;
   const u64 pinv = a.pinv[2 * l], pinvs = a.pinv[2 * l + 1], g = io.galois;
   u64 x[G::W], d[G::W], e[G::W];
-  // the combine's operands, loaded ahead of the transform where the
-  // registers hold them
+  // the combine's operands, loaded ahead of the transform where a thread has
+  // the registers: a block of 1024 threads (N = 2^13, 2^14) leaves it 128, and
+  // at 2^13 18 words went to scratch memory (20.0 us for one ciphertext of 4
+  // limbs, 16.9 with the loads after the transform; 64: 48.3, 39.8)
+  constexpr bool kAhead = G::T < 1024;
   auto load = [&] {
 #pragma unroll
     for (int k = 0; k < G::W; k++) {
@@ -1629,11 +1634,11 @@ __global__ __launch_bounds__((1 << (LOGN - LW))) void k_ring_moddown(RingModDown
       e[k] = ac[G::T * k];
     }
   };
-  if constexpr (kEarly<LW>) load();
+  if constexpr (kAhead) load();
   ring_convert<LOGN, LW>(x, a.sp.base + (2 * it + comp) * a.sp.stride, a.alpha, a.limbs, a.tab,
                          a.L, l, l, true, rt.mods, t);
   ring_forward<LOGN, LW>(x, lds, rt, l, t);
-  if constexpr (!kEarly<LW>) load();
+  if constexpr (!kAhead) load();
 #pragma unroll
   for (int k = 0; k < G::W; k++) d[k] = add_mod(d[k], pl ? pl[G::T * k] : 0, q);
 #pragma unroll
