@@ -40,7 +40,8 @@ constexpr int kMacGroupPts = 256;   // plaintexts of one launch_mac_groups
 // word for the transform; beyond 4 the separate conversion shares more
 constexpr int kRingSources = 4;
 // items per multi-rotation key inner product launch: 8 ciphertexts share a
-// key word's read where a thread's registers hold their digits
+// key word's read where a thread's registers hold their digits (k_key_inner_multi
+// has the times)
 constexpr int multi_items(int digits) { return digits <= 4 ? 8 : 4; }
 
 // Per-prime constants, resident in device memory.
@@ -396,8 +397,7 @@ struct ckks_context {
   // special limbs' conversion; environment CKKS_KS_DEFER=0 at creation keeps
   // the accumulators in HBM between the two
   bool ks_defer = true;
-  // batched key switches of at least 3 ciphertexts per part (split_count) run as
-  // `split_parts` parts, the first on the context stream and the others on
+  // batched key switches run as up to `split_parts` parts (split_count), the first on the context stream and the others on
   // `aux` streams (forked from and joined back into the context stream), so
   // that a latency-bound kernel of one part shares the CUs with a streaming
   // kernel of another; environment CKKS_SPLIT_STREAMS=<parts> at creation
@@ -612,8 +612,9 @@ void launch_convert_h4_digits(ckks_context *c, const Batch &src, const Batch &ds
                               const BCTable *const *tabs, int digits, int q_limbs, bool packed);
 void launch_rescale_lift(ckks_context *c, const Batch &last, const Batch &w, int n_items,
                          int limbs, int D, const u64 *tab);
-// N = 2^16, D <= 2 (rescale_mid_ok): launch_rescale_lift of limbs that only went through the inverse low
-// pass, into limbs that only lack the forward low pass
+// N = 2^16, D <= 2 (rescale_mid_ok): launch_rescale_lift of limbs that only
+// went through the inverse low pass, into limbs that only lack the forward low
+// pass
 bool rescale_mid_ok(const ckks_context *c, int D);
 void launch_rescale_mid(ckks_context *c, const Batch &last, const Batch &w, int n_items, int limbs,
                         int D, const u64 *tab);

@@ -1188,9 +1188,9 @@ static void ntt16_dispatch(ckks_context *c, const Batch &src, const Batch &dst, 
 // launch as long as one block's chain of loads, stages and exchanges.  The
 // two-pass radix-2 kernels this replaced exchanged after every stage (13
 // barriers, 26 us a transform of N = 2^13 in two launches, now 10.5 us for
-// fp64 primes and 12.5 us for 60-bit ones; about half of it VALU issue on the
-// block's one CU, half waits).  A key switch of 4 + 1 limbs is 5 launches
-// (350 -> 58 us), the 128 x 128 product 2792 -> 537 us.
+// fp64 primes and 12.5 us for 60-bit ones; its four waves a SIMD issue VALU
+// work for 0.55 of their life, waits take the rest).  A key switch of 4 + 1
+// limbs is 5 launches (350 -> 57 us), the 128 x 128 product 2800 -> 512 us.
 // Word positions: in the window at bit lo, word k of thread t is position
 //   (t >> lo) << (lo + LW) | k << lo | (t & (2^lo - 1)),
 // so a round's stages are on bits of k.  A thread writes back the LDS words
@@ -3423,8 +3423,8 @@ __global__ __launch_bounds__(TPB, 2) void k_convert_h4(
   // the high passes' 15 twiddles of every target's prime (forward) and every
   // source's prime (inverse), 32 words each: fp64 primes as 16 (w, w / q)
   // pairs, others as [16] psi_br and [16] Shoup constants; entry 0 is unused:
-  // word 0 holds q, word 16 floor(2^64 / q) of the others.  Each lane group works on its own primes, so these
-  // would otherwise be per-lane global loads.
+  // word 0 holds q, word 16 floor(2^64 / q) of the others.  Each lane group
+  // works on its own primes, so these would otherwise be per-lane global loads.
   u64 *ttw = tgt + (size_t)nd * TW, *stw = ttw + (size_t)nd * 32;
   // RS: the lifts, [RSD][16 rows][64 columns of the block]
   u64 *lift = stw + (size_t)ns * 32;
@@ -4480,7 +4480,12 @@ void launch_key_inner_jobs(ckks_context *c, const Strided &ext, const Strided &a
 // false: up to 8) and up to IT items, whose key words are read once.  The
 // stores of the babies and the key reads bound it: 16 ciphertexts of 25
 // limbs, 3 digits, 7 babies, 4 x 350 us with 4 items and 2 x 568 us with 8
-// (4.0 TB/s of stores and key words).
+// (4.0 TB/s of stores and key words).  Few ciphertexts lose nothing by the
+// instance for 8, whose digit count is exact: 1, 2, 4 of them, 7 babies, with a
+// 4-item instance for up to 4 digits and with this one, 12 + 12 limbs (1 digit)
+// 88 / 115 / 184 and 71 / 101 / 176 us, 24 + 12 (2) 168 / 225 / 351 and 167 /
+// 224 / 348, 26 + 8 of 59 bits (4) 318 / 388 / 526 and 291 / 351 / 488; 36 + 12
+// (3) 305 / 386 / 566 and 318 / 401 / 570.
 template <int MD, int IT, bool EXACT>
 __global__ __launch_bounds__(TPB) void k_key_inner_multi(
     Strided ext, int n_items, MultiKeys mk, int n_babies, Batch c0, const u64 *__restrict__ pmod,
@@ -4779,9 +4784,9 @@ void launch_rescale_lift(ckks_context *c, const Batch &last, const Batch &w, int
 // below 4q, so a single dropped prime costs a target one addition.  The three
 // launches it replaced wrote and read W and the dropped limbs in coefficient
 // form: 12 polynomials of 13 limbs of 59 bits 48 us, now 26 us; two dropped
-// primes of a bootstrap's 16, the lift alone 136 us, now all three 137 us.  A block takes `per` targets; parts
-// repeat the dropped limbs' work (about one target's), so that few items fill
-// the chip.  grid (16, items, parts)
+// primes of a bootstrap's 16, the lift alone 136 us, now all three 137 us.  A
+// block takes `per` targets; parts repeat the dropped limbs' work (about one
+// target's), so that few items fill the chip.  grid (16, items, parts)
 template <int D>
 __global__ __launch_bounds__(TPB) void k_rescale_mid(Batch last, Batch w, int T, int per,
                                                      const u64 *__restrict__ tab,
