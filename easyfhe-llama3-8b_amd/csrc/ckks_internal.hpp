@@ -83,11 +83,8 @@ struct PostOp {
   int plus;
 };
 
-// (both forms are read before the choice, so that a block waits for its
-// arguments once; an index past the pointers is one of a strided batch)
 __device__ __forceinline__ u64 *batch_ptr(const Batch &b, int i) {
-  u64 *p = b.p[i & (kMaxBatch - 1)];
-  return b.base ? b.base + (u64)i * b.stride : p;
+  return b.base ? b.base + (u64)i * b.stride : b.p[i];
 }
 
 // item i of a batch on the host (null for an empty batch's item 0)
@@ -397,11 +394,11 @@ struct ckks_context {
   // special limbs' conversion; environment CKKS_KS_DEFER=0 at creation keeps
   // the accumulators in HBM between the two
   bool ks_defer = true;
-  // batched key switches run as up to `split_parts` parts (split_count), the first on the context stream and the others on
-  // `aux` streams (forked from and joined back into the context stream), so
-  // that a latency-bound kernel of one part shares the CUs with a streaming
-  // kernel of another; environment CKKS_SPLIT_STREAMS=<parts> at creation
-  // (1 keeps one stream)
+  // batched key switches run as up to `split_parts` parts (split_count), the
+  // first on the context stream and the others on `aux` streams (forked from
+  // and joined back into the context stream), so that a latency-bound kernel
+  // of one part shares the CUs with a streaming kernel of another; environment
+  // CKKS_SPLIT_STREAMS=<parts> at creation (1 keeps one stream)
   static constexpr int kMaxSplit = 4;
   int split_parts = 3;
   int split_streams = 3;  // parts whose streams exist (split_parts <= this)

@@ -1188,9 +1188,9 @@ static void ntt16_dispatch(ckks_context *c, const Batch &src, const Batch &dst, 
 // launch as long as one block's chain of loads, stages and exchanges.  The
 // two-pass radix-2 kernels this replaced exchanged after every stage (13
 // barriers, 26 us a transform of N = 2^13 in two launches, now 10.5 us for
-// fp64 primes and 12.5 us for 60-bit ones; its four waves a SIMD issue VALU
-// work for 0.55 of their life, waits take the rest).  A key switch of 4 + 1
-// limbs is 5 launches (350 -> 57 us), the 128 x 128 product 2800 -> 512 us.
+// fp64 primes and 12.5 us for 60-bit ones; the block's SIMDs issue VALU work
+// for 0.55 and 0.7 of that, waits take the rest).  A key switch of 4 + 1 limbs
+// is 5 launches (350 -> 57 us), the 128 x 128 product 2800 -> 512 us.
 // Word positions: in the window at bit lo, word k of thread t is position
 //   (t >> lo) << (lo + LW) | k << lo | (t & (2^lo - 1)),
 // so a round's stages are on bits of k.  A thread writes back the LDS words
@@ -4480,7 +4480,7 @@ void launch_key_inner_jobs(ckks_context *c, const Strided &ext, const Strided &a
 // false: up to 8) and up to IT items, whose key words are read once.  The
 // stores of the babies and the key reads bound it: 16 ciphertexts of 25
 // limbs, 3 digits, 7 babies, 4 x 350 us with 4 items and 2 x 568 us with 8
-// (4.0 TB/s of stores and key words).  Few ciphertexts lose nothing by the
+// (4.0 TB/s of stores and key words).  Few ciphertexts lose little by the
 // instance for 8, whose digit count is exact: 1, 2, 4 of them, 7 babies, with a
 // 4-item instance for up to 4 digits and with this one, 12 + 12 limbs (1 digit)
 // 88 / 115 / 184 and 71 / 101 / 176 us, 24 + 12 (2) 168 / 225 / 351 and 167 /
@@ -5981,7 +5981,8 @@ __device__ u64 dbl_residue(double v, const ModQ &M) {
 // the error's residue is added: its transform is then the message's.  A block
 // takes `per` limbs: one row of 36 limbs is 256 blocks of N / 256
 // coefficients, a serial chain of limbs on one wave a SIMD (19 us), so few
-// rows are split over the limbs (11 us with the error's residues).  grid (N / 256, rows, limb parts)
+// rows are split over the limbs (11 us with the error's residues).
+// grid (N / 256, rows, limb parts)
 __global__ void k_encode_finish(const cplx *__restrict__ x, const cplx *__restrict__ twist,
                                 Batch out, int n, int logN, double scale, int total, int per,
                                 int q_limbs, int L, const ModQ *__restrict__ mods,
